@@ -90,4 +90,44 @@ int launch_wide_gemm(k3x_hip_ctx* ctx, WideKind kind, const WideGemmArgs& a, uin
 int launch_q8_rows(k3x_hip_ctx* ctx, const uint16_t* src, uint32_t rows, uint32_t cols,
                    uint32_t stride, uint16_t* q, uint32_t* qs, hipStream_t stream = nullptr);
 
+// One streaming expert GEMM launch (stream_gemm.hip).  A record names an
+// expert and its rows [off, off + rows) of the CSR order, rows > 0: {expert |
+// rows << 16, off} (recs), or the small-route grouping's {expert, rows, off,
+// -} (recs4).
+struct StreamGemmArgs {
+    const uint8_t* codes;        // MXFP4, expert 0 base of the tile array
+    const uint32_t* scales;
+    size_t codes_per_expert;     // bytes
+    size_t scales_per_expert;    // dwords
+    uint32_t kt, ks;             // K tiles (K / 128), scale dword groups
+    uint32_t nrb;                // 16-row blocks of the output (N / 16)
+    const uint16_t* a;           // activation rows, bf16
+    uint32_t a_stride;           // elements per activation row
+    uint32_t a_lo;               // split rows [hi | lo]: element offset of the lo half (0: none)
+    uint32_t a_bytes;            // bytes readable from a (loads past it read 0)
+    uint32_t gather;             // A row = pair_token[CSR row] (1) or the CSR row (0)
+    const uint4* recs4;          // null: recs
+    const uint2* recs;
+    const uint32_t* n_recs;
+    const uint32_t* pair_token;
+    const uint32_t* pair_slot;
+    uint32_t top_k;
+    uint16_t* act;               // gate/up output [row][act_stride] bf16
+    uint32_t act_stride;
+    uint32_t act_lo;             // element offset of the lo half in a row (0: none)
+    float* y;                    // down output [row][y_stride] fp32
+    uint32_t y_stride;
+    uint32_t scatter;            // y row = token * top_k + slot (1) or the CSR row (0)
+    k3x_dev::GluParams glu;
+    const uint32_t* status;
+};
+
+// Rows of one record that a workgroup multiplies at a time.
+constexpr uint32_t kStreamRows = 64;
+
+// Enqueues one launch: the records' gate/up + GLU (gateup) or down, at most
+// max_recs records of at most max_rows rows each.
+int launch_stream_gemm(k3x_hip_ctx* ctx, bool gateup, const StreamGemmArgs& a, uint32_t max_recs,
+                       uint32_t max_rows, hipStream_t stream = nullptr);
+
 }  // namespace k3x_hip

@@ -967,7 +967,7 @@ __device__ inline bool group_scan_body(
     uint32_t* __restrict__ offsets, uint32_t* __restrict__ first_use,
     uint32_t* __restrict__ n_active, uint32_t* __restrict__ active_asc,
     uint32_t* __restrict__ active_fu, uint32_t* __restrict__ witems,
-    uint32_t* __restrict__ n_witems, uint32_t chunk_rows, uint4* __restrict__ arec,
+    uint32_t* __restrict__ n_witems, uint32_t chunk_rows, uint2* __restrict__ srec,
     uint32_t* status) {
     extern __shared__ uint32_t smem[];
     uint32_t* s_cnt = smem;          // [E]
@@ -1018,14 +1018,19 @@ __device__ inline bool group_scan_body(
         const uint32_t row = (uint32_t)(pre & ((1ull << kScanItemShift) - 1));
         const uint32_t item = (uint32_t)((pre >> kScanItemShift) & ((1ull << 21) - 1));
         const uint32_t act = (uint32_t)(pre >> kScanActiveShift);
-        (void)item;
         offsets[e] = row;
         counts[e] = c;
         first_use[e] = s_fu[e];
         if (c) {
             active_asc[act] = e;
             s_alist[act] = e;
-            if (arec) arec[act] = make_uint4(e, c, row, 0u);
+            // Stream records: the expert's row chunks, in expert order (busy
+            // and idle experts mixed: some chunks bound by their weights'
+            // stream run beside others bound by their products).
+            if (srec)
+                for (uint32_t q = 0; q * chunk_rows < c; ++q)
+                    srec[item + q] = make_uint2(e | min(chunk_rows, c - q * chunk_rows) << 16,
+                                                row + q * chunk_rows);
         }
         pre += c | (uint64_t)((c + chunk_rows - 1) / chunk_rows) << kScanItemShift |
                (uint64_t)(c != 0) << kScanActiveShift;
@@ -1035,7 +1040,7 @@ __device__ inline bool group_scan_body(
     if (tid == 0) {
         offsets[E] = (uint32_t)(total & ((1ull << kScanItemShift) - 1));
         *n_active = na;
-        if (witems) *n_witems = n_items;
+        if (witems || srec) *n_witems = n_items;
     }
     if (witems) {
         // Wide GEMM work items in kWideClasses segments, one launch each:
@@ -1117,10 +1122,10 @@ __global__ __launch_bounds__(1024) void group_scan_kernel(
     uint32_t* __restrict__ offsets, uint32_t* __restrict__ first_use,
     uint32_t* __restrict__ n_active, uint32_t* __restrict__ active_asc,
     uint32_t* __restrict__ active_fu, uint32_t* __restrict__ witems,
-    uint32_t* __restrict__ n_witems, uint32_t chunk_rows, uint4* __restrict__ arec,
+    uint32_t* __restrict__ n_witems, uint32_t chunk_rows, uint2* __restrict__ srec,
     uint32_t* status) {
     (void)group_scan_body(T, K, E, chunk_cnt, chunk_fu, counts, offsets, first_use, n_active,
-                          active_asc, active_fu, witems, n_witems, chunk_rows, arec, status);
+                          active_asc, active_fu, witems, n_witems, chunk_rows, srec, status);
 }
 
 __device__ inline void group_scatter_body(uint32_t c, 
@@ -1157,12 +1162,12 @@ __global__ __launch_bounds__(1024) void group_single_kernel(
     uint32_t* __restrict__ first_use, uint32_t* __restrict__ n_active,
     uint32_t* __restrict__ active_asc, uint32_t* __restrict__ active_fu,
     uint32_t* __restrict__ witems, uint32_t* __restrict__ n_witems, uint32_t chunk_rows,
-    uint4* __restrict__ arec, uint32_t* __restrict__ pair_token, uint32_t* __restrict__ pair_slot,
+    uint2* __restrict__ srec, uint32_t* __restrict__ pair_token, uint32_t* __restrict__ pair_slot,
     uint32_t* status) {
     if (!group_count_body(0, ids, T, K, E, ready, chunk_cnt, chunk_fu, rank, status)) return;
     __syncthreads();
     if (!group_scan_body(T, K, E, chunk_cnt, chunk_fu, counts, offsets, first_use, n_active,
-                         active_asc, active_fu, witems, n_witems, chunk_rows, arec, status))
+                         active_asc, active_fu, witems, n_witems, chunk_rows, srec, status))
         return;
     __syncthreads();
     group_scatter_body(0, ids, T, K, E, chunk_cnt, rank, offsets, pair_token, pair_slot, status);
@@ -1689,6 +1694,23 @@ uint32_t wide_max_items(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K) {
     return (uint32_t)(P / k3x_hip::kWideRows + std::min<uint64_t>(d.experts, P));
 }
 
+// The streaming GEMM's records (8 bytes each) lie in the bytes of arec and
+// witems, which follow one another in the carve and which it does not use
+// itself.  Rows per record: the streaming GEMM's chunk, or the smallest
+// power of two above it at which the records fit those bytes (more than 128
+// rows an expert on average).
+uint32_t stream_max_records(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, uint32_t rows) {
+    const uint64_t P = (uint64_t)T * K;
+    return (uint32_t)(P / rows + std::min<uint64_t>(d.experts, P));
+}
+uint32_t stream_record_rows(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K) {
+    const size_t room = (((size_t)d.experts * 16 + 255) & ~(size_t)255) +
+                        (size_t)wide_max_items(d, T, K) * 4;
+    uint32_t rows = k3x_hip::kStreamRows;
+    while ((size_t)stream_max_records(d, T, K, rows) * 8 > room) rows *= 2;
+    return rows;
+}
+
 // Scratch bytes of the grouping: per-chunk counts and first uses, pair ranks.
 size_t group_scratch_bytes(uint32_t T, uint32_t K, uint32_t E) {
     const size_t tps = std::min(64u, 1024u / K), nch = (T + tps - 1) / tps;
@@ -1732,7 +1754,7 @@ size_t carve(uint8_t* base, const k3x_hip_layer_desc& d, uint32_t T, uint32_t K,
     s->xp = reinterpret_cast<uint16_t*>(s->y);
     s->sact = (uint16_t*)take((size_t)T * d.shared_inter * 2);
     s->sy = (float*)take((size_t)T * d.hidden * 4);
-    s->arec = (uint4*)take((size_t)d.experts * 16);
+    s->arec = (uint4*)take((size_t)d.experts * 16);  // witems follows: stream_record_rows
     s->witems = (uint32_t*)take((size_t)wide_max_items(d, T, K) * 4);
     s->n_witems = (uint32_t*)take(4 * (1 + k3x_hip::kWideClasses));
     s->gscratch = take(group_scratch_bytes(T, K, d.experts));
@@ -2009,11 +2031,13 @@ int launch_group(k3x_hip_ctx* ctx, const uint32_t* ids, uint32_t T, uint32_t K, 
                  uint32_t* pair_token, uint32_t* pair_slot, uint32_t* first_use,
                  uint32_t* n_active, uint32_t* active_asc, uint32_t* active_fu,
                  uint8_t* gscratch, uint32_t* witems = nullptr, uint32_t* n_witems = nullptr,
-                 uint4* arec = nullptr) {
+                 uint4* arec = nullptr, uint2* srec = nullptr,
+                 uint32_t srec_rows = 0) {
     const uint32_t tps = std::min(64u, 1024u / K), nch = (T + tps - 1) / tps;
     uint32_t* chunk_cnt = reinterpret_cast<uint32_t*>(gscratch);
     uint32_t* chunk_fu = chunk_cnt + (size_t)nch * E;
     uint8_t* rank = reinterpret_cast<uint8_t*>(chunk_fu + (size_t)nch * E);
+    const uint32_t chunk_rows = srec ? srec_rows : k3x_hip::kWideRows;
     if (!witems && T * K <= kGroupSmallPairs) {
         hipLaunchKernelGGL(group_small_kernel, dim3(1), dim3(kGroupSmallPairs), 0, ctx->stream,
                            ids, T, K, E, ready, counts, offsets, first_use, n_active, active_asc,
@@ -2025,14 +2049,14 @@ int launch_group(k3x_hip_ctx* ctx, const uint32_t* ids, uint32_t T, uint32_t K, 
                            ctx->stream, ids, T, K, E, ready, chunk_cnt, chunk_fu, rank, counts,
                            offsets,
                            first_use, n_active, active_asc, active_fu, witems, n_witems,
-                           k3x_hip::kWideRows, arec, pair_token, pair_slot, ctx->status);
+                           chunk_rows, srec, pair_token, pair_slot, ctx->status);
         return launched(ctx, 1);
     }
     hipLaunchKernelGGL(group_count_kernel, dim3(nch), dim3(1024), (size_t)(1024 + 3 * E) * 4,
                        ctx->stream, ids, T, K, E, ready, chunk_cnt, chunk_fu, rank, ctx->status);
     hipLaunchKernelGGL(group_scan_kernel, dim3(1), dim3(1024), (size_t)3 * E * 4, ctx->stream, T,
                        K, E, chunk_cnt, chunk_fu, counts, offsets, first_use, n_active, active_asc,
-                       active_fu, witems, n_witems, k3x_hip::kWideRows, arec, ctx->status);
+                       active_fu, witems, n_witems, chunk_rows, srec, ctx->status);
     hipLaunchKernelGGL(group_scatter_kernel, dim3(nch), dim3(1024), 0, ctx->stream, ids, T, K, E,
                        chunk_cnt, rank, offsets, pair_token, pair_slot, ctx->status);
     return launched(ctx, 3);
@@ -2095,6 +2119,18 @@ int run_shared_narrow(k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_hip_
     return launched(ctx, 2);
 }
 
+// The shared expert on the wide GEMM: output rows a multiple of the
+// workgroup's row blocks, K extents whole pipeline blocks.
+bool wide_shared_ok(const k3x_hip_layer_desc& d, uint32_t T) {
+    using k3x_hip::wide_rb_per_block;
+    constexpr uint32_t kq = 128 * k3x_hip::kWideStages;
+    return T >= kWideMinTokens && d.hidden % kq == 0 && d.shared_inter % kq == 0 &&
+           (d.shared_inter / 16) % wide_rb_per_block(k3x_hip::kWideSharedGateUp) == 0 &&
+           (d.hidden / 16) % wide_rb_per_block(k3x_hip::kWideSharedDown) == 0 &&
+           (uint64_t)T * std::max(d.hidden, d.shared_inter) * 2 < (1ull << 32) &&
+           (uint64_t)d.shared_inter * d.hidden * 4 < (1ull << 32);
+}
+
 // Many rows per expert: the wide grouped GEMM (128-row chunks, activations
 // staged in LDS) for the routed and the shared expert.  Shapes it needs: K
 // tile counts even, output rows a multiple of the workgroup's row blocks,
@@ -2107,14 +2143,42 @@ bool use_wide_gemm(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, bool spl
     return T >= kWideMinTokens && d.hidden % kq == 0 && d.inter % kq == 0 &&
            (d.inter / 16) % wide_rb_per_block(k3x_hip::kWideRoutedGateUp) == 0 &&
            (d.hidden / 16) % wide_rb_per_block(k3x_hip::kWideRoutedDown) == 0 &&
-           (!d.shared_inter ||
-            (d.shared_inter % kq == 0 &&
-             (d.shared_inter / 16) % wide_rb_per_block(k3x_hip::kWideSharedGateUp) == 0 &&
-             (d.hidden / 16) % wide_rb_per_block(k3x_hip::kWideSharedDown) == 0)) &&
-           rows * std::max(d.hidden, std::max(d.inter * (split ? 2 : 1), d.shared_inter)) * 2 <
-               (1ull << 32) &&
+           (!d.shared_inter || wide_shared_ok(d, T)) &&
+           rows * std::max(d.hidden, d.inter * (split ? 2 : 1)) * 2 < (1ull << 32) &&
            // weight byte offsets within one matrix pair are 32-bit as well
-           (uint64_t)std::max(d.inter, d.shared_inter) * d.hidden * 4 < (1ull << 32);
+           (uint64_t)d.inter * d.hidden * 4 < (1ull << 32);
+}
+
+// The kernels that run a call's routed experts.
+enum RoutedKind {
+    kRoutedFew,     // few tokens: the decode path's gate/up and down
+    kRoutedStream,  // the streaming GEMM (stream_gemm.hip)
+    kRoutedWide,    // many tokens: the wide GEMM (grouped_gemm.hip)
+    kRoutedNarrow,  // activation rows past 32-bit offsets: expert_gemm
+};
+
+// Tokens from which the wide GEMM's class launches beat the streaming GEMM
+// (whole layer, H=7168, 384 experts of 2048, streaming / wide: T=160 872 /
+// 1147 us, 331 1147 / 1281, 512 1484 / 1458, 768 1899 / 1773; the official
+// layer's split rows, T=331 1598 / 1867, 512 2100 / 2036).  The scaled FP4
+// path is the wide GEMM's own and keeps its range.
+constexpr uint32_t kStreamMaxTokens = 448;
+
+RoutedKind routed_kind(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank,
+                       const k3x_hip_moe_params* p) {
+    const auto& d = bank->desc;
+    const uint32_t T = p->tokens, K = p->top_k;
+    const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
+    const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
+    if (!split_in && T * K <= kGroupSmallPairs &&
+        k3x_hip::few_row_experts_eligible(ctx, bank, T, split))
+        return kRoutedFew;
+    if (!split_in && T >= (scaled_fp4(p) ? kWideMinTokens : kStreamMaxTokens) &&
+        use_wide_gemm(d, T, K, split))
+        return kRoutedWide;
+    const bool offsets = (uint64_t)T * d.hidden * (split_in ? 4 : 2) < (1ull << 32) &&
+                         (uint64_t)T * K * d.inter * (split ? 4 : 2) < (1ull << 32);
+    return offsets ? kRoutedStream : kRoutedNarrow;
 }
 
 // Arguments of the routed gate/up launch; the other three derive from them.
@@ -2302,24 +2366,26 @@ int run_wide(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     return st ? st : jst;
 }
 
+// The shared expert on `stream` (stage marks only on the context stream).
+int run_shared(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
+               const Scratch& s, const uint16_t* xn, const GluParams& glu, hipStream_t stream) {
+    const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
+    return !split_in && wide_shared_ok(bank->desc, p->tokens)
+               ? run_shared_wide(ctx, bank, p, s, xn, glu, stream)
+               : run_shared_narrow(ctx, bank, p, s, xn, glu, split_in, stream);
+}
+
 // Grouping, expert GEMMs, shared expert, combine.  xn is the bf16 input of
 // the experts; ids/weights [T][K] device.
-// Whether a call's shared expert runs on the context's second stream: the
-// wide path (the routed GEMMs run for milliseconds) and the verification
-// windows on the decode kernels (hundreds of microseconds of routed
-// streaming beside a few dozen shared workgroups).  With stage profiling on,
-// everything stays on the context stream.
+// Whether a call's shared expert runs on the context's second stream: past
+// the few-token calls, where the routed experts stream for hundreds of
+// microseconds or more beside it.  With stage profiling on, everything stays
+// on the context stream.
 bool shared_on_side(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_hip_moe_params* p) {
-    const auto& d = bank->desc;
-    const uint32_t T = p->tokens, K = p->top_k;
-    const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
-    const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
-    const bool wide_path = !split_in && use_wide_gemm(d, T, K, split);
-    const bool chunked_rows = !wide_path && !split_in && T > k3x_hip::kMaxDecodeTokens &&
-                              T <= k3x_hip::kChunkedMaxTokens &&
-                              k3x_hip::few_row_experts_eligible(ctx, bank,
-                                                                k3x_hip::kMaxDecodeTokens, split);
-    return (wide_path || chunked_rows) && d.shared_inter && !ctx->profiling && ctx->side_stream;
+    const RoutedKind kind = routed_kind(ctx, bank, p);
+    return bank->desc.shared_inter && !ctx->profiling && ctx->side_stream &&
+           (kind == kRoutedWide ||
+            (kind == kRoutedStream && p->tokens > (uint32_t)k3x_hip::kMaxDecodeTokens));
 }
 
 // Launches the shared expert on the second stream after the context
@@ -2327,16 +2393,10 @@ bool shared_on_side(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_
 // stream joins on.
 int fork_shared(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
                 const Scratch& s, const uint16_t* xn, const GluParams& glu) {
-    const auto& d = bank->desc;
-    const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
-    const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
-    const bool wide_path = !split_in && use_wide_gemm(d, p->tokens, p->top_k, split);
     if (hipEventRecord(ctx->fork_ev, ctx->stream) != hipSuccess ||
         hipStreamWaitEvent(ctx->side_stream, ctx->fork_ev, 0) != hipSuccess)
         return K3X_ERR_BACKEND_UNAVAILABLE;
-    const int sst = wide_path ? run_shared_wide(ctx, bank, p, s, xn, glu, ctx->side_stream)
-                              : run_shared_narrow(ctx, bank, p, s, xn, glu, split_in,
-                                                  ctx->side_stream);
+    const int sst = run_shared(ctx, bank, p, s, xn, glu, ctx->side_stream);
     if (hipEventRecord(ctx->join_ev, ctx->side_stream) != hipSuccess) {
         // Without the event, order the streams the blunt way.
         (void)hipStreamSynchronize(ctx->side_stream);
@@ -2354,24 +2414,16 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     const auto& d = bank->desc;
     const uint32_t T = p->tokens, K = p->top_k;
     GluParams glu{(int)p->glu, p->situ_beta, (int)p->has_situ_linear, p->situ_linear_beta};
-    // Wide path with a shared expert: its GEMMs depend only on xn, so they
-    // go to the side stream now and run beside the grouping and the routed
-    // GEMMs (filling the small grouping launches and the routed GEMMs'
-    // tails); the context stream waits for them before the combine, and on
-    // every early return (they read and write this call's scratch).  With
-    // stage profiling on, everything stays on the context stream.
+    // The shared expert's GEMMs depend only on xn, so past the few-token
+    // calls they go to the side stream now and run beside the grouping and
+    // the routed GEMMs (filling the small grouping launches and the routed
+    // GEMMs' tails); the context stream waits for them before the combine,
+    // and on every early return (they read and write this call's scratch).
+    // With stage profiling on, everything stays on the context stream.
     const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
-    // Split input rows [hi | lo] (2 H): the narrow GEMMs, gate/up over both
-    // halves.
+    // Split input rows [hi | lo] (2 H): gate/up over both halves.
     const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
-    const bool wide_path = !split_in && use_wide_gemm(d, T, K, split);
-    // Verification windows on the decode kernels (below): the routed experts
-    // stream for hundreds of microseconds, the shared expert's narrow GEMMs
-    // run a few dozen workgroups; on the side stream they overlap.
-    const bool chunked_rows = !wide_path && !split_in && T > k3x_hip::kMaxDecodeTokens &&
-                              T <= k3x_hip::kChunkedMaxTokens &&
-                              k3x_hip::few_row_experts_eligible(ctx, bank,
-                                                                k3x_hip::kMaxDecodeTokens, split);
+    const RoutedKind kind = routed_kind(ctx, bank, p);
     const bool side = shared_on_side(ctx, bank, p);
     struct Join {
         k3x_hip_ctx* ctx;
@@ -2393,37 +2445,93 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
         }
     }
     int mark = begin_stage(ctx, K3X_STAGE_GROUP);
-    // Work items of the wide GEMM only where it runs (without them a small
-    // route is grouped by one workgroup).
-    // Few tokens: the routed experts on the decode path's kernels, fed by
-    // the active-slot records of the small-route grouping.
-    // Up to kChunkedMaxTokens tokens (verification windows): the same
-    // kernels over slots of any size, rows through LDS a few at a time.
-    const bool few = !wide_path && !split_in && T * K <= kGroupSmallPairs &&
-                     k3x_hip::few_row_experts_eligible(ctx, bank, T, split);
-    const bool chunked = !few && chunked_rows;
+    // The wide GEMM takes work items, the streaming one records: row chunks
+    // (srec), or one an active expert from the small-route grouping (arec;
+    // the decode path's kernels read the same records).
+    const bool small = kind != kRoutedWide && T * K <= kGroupSmallPairs;
+    const bool chunks = kind == kRoutedStream && !small;
+    const uint32_t srec_rows = stream_record_rows(d, T, K);
+    uint2* const srec = reinterpret_cast<uint2*>(s.arec);
     // A route grouped with its Top-K (topk_group_kernel) holds what the
     // small-route grouping below would write: no wide path there.
-    if (s.grouped && (wide_path || T * K > kGroupSmallPairs)) return K3X_ERR_INVALID_EXTENT;
+    if (s.grouped && !small) return K3X_ERR_INVALID_EXTENT;
     int st = s.grouped ? K3X_OK
                        : launch_group(ctx, ids, T, K, d.experts, bank->ready_dev, s.counts,
                                       s.offsets, s.pair_token, s.pair_slot, s.first_use,
                                       s.n_active, s.active_asc, s.active_fu, s.gscratch,
-                                      wide_path ? s.witems : nullptr,
-                                      wide_path ? s.n_witems : nullptr,
-                                      few || chunked ? s.arec : nullptr);
+                                      kind == kRoutedWide ? s.witems : nullptr, s.n_witems,
+                                      small ? s.arec : nullptr, chunks ? srec : nullptr,
+                                      srec_rows);
     end_stage(ctx, mark);
     if (st) return st;
     const uint32_t max_active = std::min<uint32_t>(d.experts, T * K);
-    const bool wide = T > 16;  // more than one 16-row MFMA tile per expert possible
-    if (wide_path) {
+    if (kind == kRoutedWide) {
         if ((st = run_wide(ctx, bank, p, s, xn, glu, !side))) return st;
         if ((st = joiner.join())) return st;
         return k3x_hip::launch_combine(ctx, s.y, weights, d.shared_inter ? s.sy : nullptr, K,
                                        d.hidden, T, out, out_f32,
                                        (p->flags & K3X_FLAG_ROUND_EXPERT_OUT) != 0);
     }
-
+    if (kind == kRoutedStream) {
+        k3x_hip::StreamGemmArgs g{};
+        g.codes = bank->gu_codes;
+        g.scales = bank->gu_scales;
+        g.codes_per_expert = bank->gu_codes_per_expert;
+        g.scales_per_expert = bank->gu_scales_per_expert;
+        g.kt = bank->gate.kt;
+        g.ks = bank->gate.ks;
+        g.nrb = d.inter / 16;
+        g.a = xn;
+        g.a_stride = split_in ? 2 * d.hidden : d.hidden;
+        g.a_lo = split_in ? d.hidden : 0;
+        g.a_bytes = T * g.a_stride * 2;
+        g.gather = 1;
+        g.recs4 = small ? s.arec : nullptr;
+        g.recs = srec;
+        g.n_recs = small ? s.n_active : s.n_witems;
+        g.pair_token = s.pair_token;
+        g.pair_slot = s.pair_slot;
+        g.top_k = K;
+        g.act = s.act;
+        g.act_stride = split ? 2 * d.inter : d.inter;
+        g.act_lo = split ? d.inter : 0;
+        g.glu = glu;
+        g.status = ctx->status;
+        // An expert takes at most one row a token.
+        const uint32_t recs = small ? max_active : stream_max_records(d, T, K, srec_rows);
+        const uint32_t rec_rows = small ? T : std::min(T, srec_rows);
+        mark = begin_stage(ctx, K3X_STAGE_GATE_UP);
+        st = k3x_hip::launch_stream_gemm(ctx, true, g, recs, rec_rows);
+        end_stage(ctx, mark);
+        if (st) return st;
+        g.codes = bank->dn_codes;
+        g.scales = bank->dn_scales;
+        g.codes_per_expert = bank->dn_codes_per_expert;
+        g.scales_per_expert = bank->dn_scales_per_expert;
+        g.kt = bank->down.kt;
+        g.ks = bank->down.ks;
+        g.nrb = d.hidden / 16;
+        g.a = s.act;
+        g.a_stride = g.act_stride;
+        g.a_lo = g.act_lo;
+        g.a_bytes = T * K * g.act_stride * 2;
+        g.gather = 0;
+        g.y = s.y;
+        g.y_stride = d.hidden;
+        g.scatter = 1;
+        mark = begin_stage(ctx, K3X_STAGE_DOWN);
+        st = k3x_hip::launch_stream_gemm(ctx, false, g, recs, rec_rows);
+        end_stage(ctx, mark);
+        if (st) return st;
+        if (d.shared_inter && !side &&
+            (st = run_shared(ctx, bank, p, s, xn, glu, ctx->stream)))
+            return st;
+        if ((st = joiner.join())) return st;
+        return k3x_hip::launch_combine(ctx, s.y, weights, d.shared_inter ? s.sy : nullptr, K,
+                                       d.hidden, T, out, out_f32,
+                                       (p->flags & K3X_FLAG_ROUND_EXPERT_OUT) != 0);
+    }
+    const bool few = kind == kRoutedFew;
     GemmArgs g{};
     g.status = ctx->status;
     g.glu = glu;
@@ -2449,13 +2557,10 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     g.act_stride = split ? 2 * d.inter : d.inter;
     g.act_lo = split ? d.inter : 0;
     mark = begin_stage(ctx, K3X_STAGE_GATE_UP);
-    if (few || chunked) {
-        if ((st = k3x_hip::launch_few_row_gate_up(ctx, bank, T, K, s, xn, glu, split, chunked)))
-            return st;
-    } else if (wide) {
-        launch_gemm<true, true, 4, 1>(ctx, g, max_active, d.inter);
+    if (few) {
+        if ((st = k3x_hip::launch_few_row_gate_up(ctx, bank, T, K, s, xn, glu, split))) return st;
     } else {
-        launch_gemm<true, true, 1, 1>(ctx, g, max_active, d.inter);
+        launch_gemm<true, true, 4, 1>(ctx, g, max_active, d.inter);
     }
     end_stage(ctx, mark);
     // Routed down, scattered to [token][slot].
@@ -2477,28 +2582,26 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     // fused mix), after the shared expert, whose output it adds.
     if (few && k3x_hip::few_row_mix_eligible(bank, T)) {
         if (d.shared_inter && !side &&
-            (st = run_shared_narrow(ctx, bank, p, s, xn, glu, split_in, ctx->stream)))
+            (st = run_shared(ctx, bank, p, s, xn, glu, ctx->stream)))
             return st;
         if ((st = joiner.join())) return st;
         const k3x_hip::FewRowMix mix{weights, d.shared_inter ? s.sy : nullptr, out, out_f32,
                                      (p->flags & K3X_FLAG_ROUND_EXPERT_OUT) != 0};
         mark = begin_stage(ctx, K3X_STAGE_DOWN);
-        st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split, false, &mix);
+        st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split, &mix);
         end_stage(ctx, mark);
         return st;
     }
     mark = begin_stage(ctx, K3X_STAGE_DOWN);
-    if (few || chunked) {
-        if ((st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split, chunked))) return st;
-    } else if (wide) {
-        launch_gemm<true, false, 4, 2>(ctx, dn, max_active, d.hidden);
+    if (few) {
+        if ((st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split))) return st;
     } else {
-        launch_gemm<true, false, 1, 2>(ctx, dn, max_active, d.hidden);
+        launch_gemm<true, false, 4, 2>(ctx, dn, max_active, d.hidden);
     }
     end_stage(ctx, mark);
-    if ((st = launched(ctx, few || chunked ? 0 : 2))) return st;
+    if ((st = launched(ctx, few ? 0 : 2))) return st;
     if (d.shared_inter && !side &&
-        (st = run_shared_narrow(ctx, bank, p, s, xn, glu, split_in, ctx->stream)))
+        (st = run_shared(ctx, bank, p, s, xn, glu, ctx->stream)))
         return st;
     if ((st = joiner.join())) return st;
     return k3x_hip::launch_combine(ctx, s.y, weights, d.shared_inter ? s.sy : nullptr, K,
