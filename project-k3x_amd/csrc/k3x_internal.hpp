@@ -250,23 +250,18 @@ int launch_topk(k3x_hip_ctx* ctx, const float* logits, const float* bias, uint32
 // running over both halves: an fp32 activation into the bf16 MFMA.
 int dense_gate_up(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t I, uint32_t H, const uint16_t* x,
                   uint32_t T, const k3x_dev::GluParams& glu, uint16_t* act, hipStream_t stream,
-                  bool split = false);
-// Up to kDenseDirectTokens rows the projections run as a split-K GEMV on
-// any stream, and dense_down can round its output to bf16 itself (y_bf16;
-// y is then unused); above, y_bf16 must be null, and the projections run on
-// the wide GEMM (any stream) where its shape rules allow, else on the narrow
-// GEMM (the context stream only).
-constexpr uint32_t kDenseDirectTokens = 16;
-// True when both projections of a dense GLU MLP (gate/up I x H, down H x I)
-// may be enqueued on a stream other than the context's for T rows.
-bool dense_mlp_any_stream(uint32_t I, uint32_t H, uint32_t T);
-// True when dense_down of an N x K projection over T rows may be enqueued on
-// a stream other than the context's.
-bool dense_down_any_stream(uint32_t N, uint32_t K, uint32_t T);
+                  bool split = false, bool split_in = false);
+// split_in: x rows [hi | lo] of 2 H, gate and up over both halves.
+// Few rows run as a split-K GEMV, more on the rows kernel, many on the wide
+// GEMM where its shape rules allow; all on any stream.  The first two
+// (dense_direct) can round dense_down's output to bf16 themselves (y_bf16; y
+// is then unused) and write the official layer's output (dense_down_output);
+// on the wide GEMM y_bf16 must be null.
+bool dense_direct(uint32_t N, uint32_t K, uint32_t T);
 int dense_down(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K, const uint16_t* a,
                uint32_t T, float* y, hipStream_t stream, uint16_t* y_bf16 = nullptr,
                bool split = false);
-// Up to kDenseDirectTokens rows on the context stream: y = tiles . a with the
+// dense_direct rows on the context stream: y = tiles . a with the
 // official layer's output in the epilogue: routed = y (fp32) and out =
 // bf16(bf16(prefix) + bf16(bf16(y) + bf16(shared))) (shared may be null).
 int dense_down_output(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K,

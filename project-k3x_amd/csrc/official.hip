@@ -802,20 +802,17 @@ int k3x_hip_official_ffn(k3x_hip_ctx* ctx, k3x_hip_official* o, const k3x_hip_mo
     // Shared FFN on hidden (official_moe.cpp:105-117, :307): on the side
     // stream beside the route and the experts (few rows: the routed kernels
     // leave the device half idle; many rows: the latency-bound route steps
-    // and the experts' tails do), joined before the output; in line when
-    // its projections cannot leave the context stream.
+    // and the experts' tails do), joined before the output.
     // Few tokens with the route found here: the route, the latent projection
     // and the shared FFN in two launches on the context stream (the
     // projections' workgroups beside the route's), no second stream.
     const bool fused = !ids && o->bank->desc.experts == o->E &&
                        k3x_hip::official_decode_eligible(o->E, o->H, o->L, o->I_s, K, T);
-    const bool side = !fused && o->I_s && ctx->side_stream && !ctx->profiling &&
-                      k3x_hip::dense_mlp_any_stream(o->I_s, o->H, T);
+    const bool side = !fused && o->I_s && ctx->side_stream && !ctx->profiling;
     // The latent projection needs hidden only: with the route found here it
     // goes first on the side stream, beside the route's latency-bound
     // launches, and the experts wait for it alone.
-    const bool latent_side = !fused && !ids && ctx->side_stream && !ctx->profiling &&
-                             k3x_hip::dense_down_any_stream(o->L, o->H, T);
+    const bool latent_side = !fused && !ids && ctx->side_stream && !ctx->profiling;
     struct Join {
         k3x_hip_official* o;
         bool armed = false;
@@ -839,10 +836,10 @@ int k3x_hip_official_ffn(k3x_hip_ctx* ctx, k3x_hip_official* o, const k3x_hip_mo
         return r ? r : k3x_hip::dense_down(ctx, o->shared_dn, o->H, o->I_s, b.sact, T, b.shared,
                                            stream, nullptr, true);
     };
-    // latent = bf16(routed_down . hidden) (official_moe.cpp:305); few rows
-    // round in the GEMV's own epilogue.
+    // latent = bf16(routed_down . hidden) (official_moe.cpp:305), rounded in
+    // the projection's own epilogue where that can.
     auto latent = [&](hipStream_t stream) {
-        if (T <= k3x_hip::kDenseDirectTokens)
+        if (k3x_hip::dense_direct(o->L, o->H, T))
             return k3x_hip::dense_down(ctx, o->routed_down, o->L, o->H, hidden, T, nullptr, stream,
                                        b.latent);
         const int r = k3x_hip::dense_down(ctx, o->routed_down, o->L, o->H, hidden, T,
@@ -926,7 +923,7 @@ int k3x_hip_official_ffn(k3x_hip_ctx* ctx, k3x_hip_official* o, const k3x_hip_mo
                                                   o->routed_norm, p->rms_epsilon, T, prefix,
                                                   o->I_s ? b.shared : nullptr, b.routed, out);
         if (st) return st;
-    } else if (T <= k3x_hip::kDenseDirectTokens) {
+    } else if (k3x_hip::dense_direct(o->H, o->L, T)) {
         // Few rows: the output formula in the routed_up GEMV's epilogue, after
         // the shared FFN (long finished on the side stream by now).
         if (!st && o->I_s && !side && !fused) st = shared_ffn(ctx->stream);

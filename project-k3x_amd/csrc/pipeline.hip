@@ -1198,48 +1198,38 @@ struct GemmArgs {
     uint32_t a_stride;          // elements per activation row
     uint32_t a_lo;              // split rows [hi | lo]: element offset of the lo half (0: none)
     uint32_t gather;            // A row = pair_token[off+m] (1) or off+m (0)
-    const uint32_t* n_active;   // grouping (nullptr = single block of `tokens` rows)
+    const uint32_t* n_active;
     const uint32_t* active;
     const uint32_t* counts;
     const uint32_t* offsets;
     const uint32_t* pair_token;
     const uint32_t* pair_slot;
-    uint32_t tokens;
     uint32_t top_k;
     uint16_t* act;              // GATEUP output [row][act_stride] bf16
     uint32_t act_stride;
     uint32_t act_lo;            // GATEUP: element offset of the lo half in a row (0: none)
-    float* y;                   // down output [row][y_stride] fp32
+    float* y;                   // down output [token * top_k + slot][y_stride] fp32
     uint32_t y_stride;
-    uint32_t scatter;           // y row = token*top_k + slot (1) or off+m (0)
     GluParams glu;
     const uint32_t* status;
 };
 
-constexpr int kGemmDepth = 4;  // K steps in flight per wave of a one-row-tile GEMM
-
 // SPLIT: activation rows [hi | lo] (a_lo elements apart), an fp32 value in
 // two bf16 halves; each weight fragment meets both (two MFMAs, the weights
 // read once).
-template <bool FP4, bool GATEUP, int MT, int NT, bool SPLIT>
+template <bool GATEUP, int MT, int NT, bool SPLIT>
 __global__ __launch_bounds__(256) void expert_gemm(GemmArgs a) {
     if (*(volatile const uint32_t*)a.status) return;
     const uint32_t eb = blockIdx.x / a.blocks_per_expert;
     const uint32_t jb = blockIdx.x % a.blocks_per_expert;
-    uint32_t e = 0, cnt = a.tokens, off = 0;
-    if (a.active) {
-        if (eb >= *a.n_active) return;
-        e = a.active[eb];
-        cnt = a.counts[e];
-        off = a.offsets[e];
-    }
+    if (eb >= *a.n_active) return;
+    const uint32_t e = a.active[eb], cnt = a.counts[e], off = a.offsets[e];
     constexpr int S = GATEUP ? 2 : 1;  // tiles per row block and K step
-    constexpr int U = FP4 ? 1 : 4;     // 16-byte words per lane per tile
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int g = lane >> 4, n = lane & 15;
     const uint32_t rb0 = (jb * 4 + wave) * NT;
     const uint4* codes = reinterpret_cast<const uint4*>(a.codes + e * a.codes_per_expert);
-    const uint32_t* scales = FP4 ? a.scales + e * a.scales_per_expert : nullptr;
+    const uint32_t* scales = a.scales + e * a.scales_per_expert;
     constexpr int H2 = SPLIT ? 2 : 1;  // activation halves
 
     for (uint32_t m0 = 0; m0 < cnt; m0 += 16 * MT) {
@@ -1264,67 +1254,46 @@ __global__ __launch_bounds__(256) void expert_gemm(GemmArgs a) {
 #pragma unroll
                 for (int w = 0; w < S; ++w) acc[mt][nt][w] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-        // One row tile: D K steps of loads issued together (steps past the
-        // last tile clamped, their activations zeroed), since a lone step's
-        // round trip would bound the wave.
-        constexpr int D = MT == 1 ? kGemmDepth : 1;
-        for (uint32_t k0 = 0; k0 < a.kt; k0 += D) {
-            uint4 bt[D][NT][S][U];
-            float sc[D][NT][S];
-            bf16x8 af[D][MT][H2][4];
+        for (uint32_t k = 0; k < a.kt; ++k) {
+            uint4 bt[NT][S];
+            float sc[NT][S];
+            bf16x8 af[MT][H2][4];
 #pragma unroll
-            for (int d = 0; d < D; ++d) {
-                const uint32_t k = min(k0 + d, a.kt - 1);
+            for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                for (int w = 0; w < S; ++w) {
+                    bt[nt][w] = codes[(((size_t)(rb0 + nt) * a.kt + k) * S + w) * 64 + lane];
+                    const uint32_t sw =
+                        scales[(((size_t)(rb0 + nt) * a.ks + k / 4) * S + w) * 64 + lane];
+                    sc[nt][w] = e8m0_to_f32((sw >> (8 * (k & 3))) & 0xffu);
+                }
+#pragma unroll
+            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                for (int h = 0; h < H2; ++h) {
+                    const uint4* p = reinterpret_cast<const uint4*>(
+                        arow[mt] + (h ? a.a_lo : 0u) + (size_t)k * 128);
+#pragma unroll
+                    for (int j = 0; j < 4; ++j) {
+                        const uint4 v = p[j];
+                        af[mt][h][j] = as_bf16x8(live[mt] ? v : make_uint4(0, 0, 0, 0));
+                    }
+                }
+#pragma unroll
+            for (int j = 0; j < 4; ++j)
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                     for (int w = 0; w < S; ++w) {
-                        const size_t base = (((size_t)(rb0 + nt) * a.kt + k) * S + w) * U * 64 + lane;
+                        const uint4 c = bt[nt][w];
+                        const uint32_t word = j == 0 ? c.x : j == 1 ? c.y : j == 2 ? c.z : c.w;
+                        const bf16x8 b = dequant8(word, sc[nt][w]);
 #pragma unroll
-                        for (int u = 0; u < U; ++u) bt[d][nt][w][u] = codes[base + u * 64];
-                        if constexpr (FP4) {
-                            const uint32_t sw =
-                                scales[(((size_t)(rb0 + nt) * a.ks + k / 4) * S + w) * 64 + lane];
-                            sc[d][nt][w] = e8m0_to_f32((sw >> (8 * (k & 3))) & 0xffu);
-                        }
+                        for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                            for (int h = 0; h < H2; ++h)
+                                acc[mt][nt][w] = mfma16x16x32(af[mt][h][j], b, acc[mt][nt][w]);
                     }
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int h = 0; h < H2; ++h) {
-                        const uint4* p = reinterpret_cast<const uint4*>(
-                            arow[mt] + (h ? a.a_lo : 0u) + (size_t)k * 128);
-                        const bool use = live[mt] && k0 + d < a.kt;
-#pragma unroll
-                        for (int j = 0; j < 4; ++j) {
-                            const uint4 v = p[j];
-                            af[d][mt][h][j] = as_bf16x8(use ? v : make_uint4(0, 0, 0, 0));
-                        }
-                    }
-            }
-#pragma unroll
-            for (int d = 0; d < D; ++d)
-#pragma unroll
-                for (int j = 0; j < 4; ++j) {
-#pragma unroll
-                    for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                        for (int w = 0; w < S; ++w) {
-                            bf16x8 b;
-                            if constexpr (FP4) {
-                                const uint4 c = bt[d][nt][w][0];
-                                const uint32_t word = j == 0 ? c.x : j == 1 ? c.y : j == 2 ? c.z : c.w;
-                                b = dequant8(word, sc[d][nt][w]);
-                            } else {
-                                b = as_bf16x8(bt[d][nt][w][j]);
-                            }
-#pragma unroll
-                            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                                for (int h = 0; h < H2; ++h)
-                                    acc[mt][nt][w] = mfma16x16x32(af[d][mt][h][j], b, acc[mt][nt][w]);
-                        }
-                }
         }
 
 #pragma unroll
@@ -1344,9 +1313,7 @@ __global__ __launch_bounds__(256) void expert_gemm(GemmArgs a) {
                         if (a.act_lo) dst[a.act_lo] = act_lo_bf16(v, hi);
                     } else {
                         const uint32_t r = off + row;
-                        const size_t yrow = a.scatter
-                                                ? (size_t)a.pair_token[r] * a.top_k + a.pair_slot[r]
-                                                : (size_t)r;
+                        const size_t yrow = (size_t)a.pair_token[r] * a.top_k + a.pair_slot[r];
                         a.y[yrow * a.y_stride + col] = acc[mt][nt][0][i];
                     }
                 }
@@ -1366,7 +1333,7 @@ __global__ __launch_bounds__(256) void expert_gemm(GemmArgs a) {
 // stored in fp32 (runtime/src/official_moe.cpp:336-340).
 // ---------------------------------------------------------------------------
 constexpr int kGemvWaves = 16;
-constexpr uint32_t kGemvMaxTokens = k3x_hip::kDenseDirectTokens;
+constexpr uint32_t kGemvMaxTokens = 16;
 
 // Weight tiles are read once a call: non-temporal loads (the lines are not
 // kept in L2 / MALL), which stream faster than cached ones (the official
@@ -1401,6 +1368,28 @@ struct GemvArgs {
     const float* gamma;
     float eps;
 };
+
+// Output element `at` of a dense projection from its fp32 sums (gate and up
+// for OUT 2): 0 fp32, 1 bf16, 2 GLU -> bf16 (and its lo half), 3 the official
+// layer's output formula.
+template <int OUT, int S>
+__device__ __forceinline__ void store_dense(const GemvArgs& a, size_t at, const float (&v)[S]) {
+    if constexpr (OUT == 0) static_cast<float*>(a.out)[at] = v[0];
+    else if constexpr (OUT == 1) static_cast<uint16_t*>(a.out)[at] = f32_to_bf16(v[0]);
+    else if constexpr (OUT == 2) {
+        const float g = glu(v[0], v[S - 1], a.glu);
+        const uint16_t hi = f32_to_bf16(g);
+        static_cast<uint16_t*>(a.out)[at] = hi;
+        if (a.out_lo) static_cast<uint16_t*>(a.out)[at + a.out_lo] = act_lo_bf16(g, hi);
+    }
+    else {
+        auto r16 = [](float x) { return __uint_as_float((uint32_t)f32_to_bf16(x) << 16); };
+        a.routed[at] = v[0];
+        const float sh = a.shared ? r16(a.shared[at]) : 0.0f;
+        const float combined = r16(__fadd_rn(r16(v[0]), sh));
+        static_cast<uint16_t*>(a.out)[at] = f32_to_bf16(__fadd_rn(r16(a.prefix[at]), combined));
+    }
+}
 
 // NORM: tokens a workgroup normalises (256 threads each) and 16-byte chunks
 // of the raw rows and of gamma its threads load (two and one a thread).
@@ -1578,28 +1567,94 @@ __device__ __forceinline__ void dense_gemv_body(const GemvArgs& a, uint32_t rb) 
 #pragma unroll
         for (int q = 1; q < W; ++q) v[w] = __fadd_rn(v[w], part[q][w][pl][pi]);
     }
-    const size_t at = (size_t)t * a.out_stride + (size_t)rb * 16 + c;
-    if constexpr (OUT == 0) static_cast<float*>(a.out)[at] = v[0];
-    else if constexpr (OUT == 1) static_cast<uint16_t*>(a.out)[at] = f32_to_bf16(v[0]);
-    else if constexpr (OUT == 2) {
-        const float g = glu(v[0], v[S - 1], a.glu);
-        const uint16_t hi = f32_to_bf16(g);
-        static_cast<uint16_t*>(a.out)[at] = hi;
-        if (a.out_lo) static_cast<uint16_t*>(a.out)[at + a.out_lo] = act_lo_bf16(g, hi);
-    }
-    else {
-        auto r16 = [](float x) { return __uint_as_float((uint32_t)f32_to_bf16(x) << 16); };
-        a.routed[at] = v[0];
-        const float sh = a.shared ? r16(a.shared[at]) : 0.0f;
-        const float combined = r16(__fadd_rn(r16(v[0]), sh));
-        static_cast<uint16_t*>(a.out)[at] = f32_to_bf16(__fadd_rn(r16(a.prefix[at]), combined));
-    }
+    store_dense<OUT, S>(a, (size_t)t * a.out_stride + (size_t)rb * 16 + c, v);
 }
 
 template <int S, int D, int OUT, int W = kGemvWaves, bool SPLIT = false, bool LDSX = false,
           bool NORM = false>
 __global__ __launch_bounds__(64 * W) void dense_gemv_kernel(GemvArgs a) {
     dense_gemv_body<S, D, OUT, W, SPLIT, LDSX, NORM>(a, blockIdx.x);
+}
+
+// The dense projections of more rows than the GEMV's: NB blocks of 16 output
+// rows (pairs, S = 2) x 16 MT tokens per 1024-thread workgroup, its 16 waves
+// over the K tiles (wave w takes tiles w, w + 16, ...), the partial
+// accumulators summed in wave order through LDS.  Each weight fragment meets
+// the MT row tiles; the activations come from the L2, which holds them for
+// every workgroup.
+// Bound: latency (a wave streams two to four tiles), then the L2's rate as
+// the tokens grow (every workgroup reads all of its tokens' rows: NB = 2
+// halves that for the single matrices).  K is split inside the workgroup
+// because 128 to 448 row blocks are all the workgroups such a matrix has, and
+// the narrow GEMM's full-K waves (28 to 96 workgroups) left most of the chip
+// idle.  OUT, split rows and epilogues as dense_gemv_body.
+constexpr int kRowsWaves = 16;
+
+template <int S, int NB, int MT, int OUT, bool SPLIT>
+__global__ __launch_bounds__(64 * kRowsWaves) void dense_rows_kernel(GemvArgs a) {
+    __shared__ f32x4 part[kRowsWaves][MT][NB * S][64];
+    if (*(volatile const uint32_t*)a.status) return;
+    const int lane = threadIdx.x & 63;
+    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t g = lane >> 4, n = lane & 15;
+    const uint32_t rb = blockIdx.x * NB, m0 = blockIdx.y * (16 * MT);
+    constexpr int H2 = SPLIT ? 2 : 1;  // activation halves
+    const u32x4* xr[MT];               // rows past the last repeat it (not stored)
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+        xr[mt] = reinterpret_cast<const u32x4*>(
+            a.x + (size_t)min(m0 + 16 * mt + n, a.tokens - 1) * a.x_stride + 32 * g);
+    const u32x4* wt = reinterpret_cast<const u32x4*>(a.tiles) + (size_t)rb * a.kt * S * 256 + lane;
+    f32x4 acc[MT][NB * S];
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int w = 0; w < NB * S; ++w) acc[mt][w] = f32x4{0.f, 0.f, 0.f, 0.f};
+    for (uint32_t k = wave; k < a.kt; k += kRowsWaves) {
+        u32x4 b[NB * S][4];
+#pragma unroll
+        for (int w = 0; w < NB * S; ++w)
+#pragma unroll
+            for (int u = 0; u < 4; ++u)
+                b[w][u] = wt[(((size_t)(w / S) * a.kt + k) * S + w % S) * 256 + u * 64];
+#pragma unroll
+        for (int h = 0; h < H2; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                u32x4 xv[MT];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+                    xv[mt] = xr[mt][(size_t)k * 16 + j + (h ? a.x_lo / 8 : 0)];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int w = 0; w < NB * S; ++w)
+                        acc[mt][w] = mfma16x16x32(as_bf16x8(xv[mt]), as_bf16x8(b[w][j]),
+                                                  acc[mt][w]);
+            }
+    }
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+        for (int w = 0; w < NB * S; ++w) part[wave][mt][w][lane] = acc[mt][w];
+    __syncthreads();
+    // Thread 16 r + c finishes row r of the chunk, column c of each block:
+    // lane 16 (r % 16 / 4) + c, element r % 4 of row tile r / 16.
+    const uint32_t r = threadIdx.x / 16, c = threadIdx.x % 16, t = m0 + r;
+    if (r >= 16 * MT || t >= a.tokens) return;
+    const uint32_t pl = 16 * (r % 16 / 4) + c, pi = r % 4, pm = r / 16;
+#pragma unroll
+    for (int i = 0; i < NB; ++i) {
+        float v[S];
+#pragma unroll
+        for (int w = 0; w < S; ++w) {
+            v[w] = part[0][pm][i * S + w][pl][pi];
+#pragma unroll
+            for (int q = 1; q < kRowsWaves; ++q)
+                v[w] = __fadd_rn(v[w], part[q][pm][i * S + w][pl][pi]);
+        }
+        store_dense<OUT, S>(a, (size_t)t * a.out_stride + (size_t)(rb + i) * 16 + c, v);
+    }
 }
 
 // ---------------------------------------------------------------------------
@@ -1682,8 +1737,10 @@ using Scratch = k3x_hip::LayerBuffers;
 using k3x_hip::begin_stage;
 using k3x_hip::end_stage;
 
-// Tokens from which the general path runs the wide grouped GEMM.
+// Tokens from which the wide grouped GEMM takes routed experts at all, and
+// dense projections.
 constexpr uint32_t kWideMinTokens = 128;
+constexpr uint32_t kDenseWideTokens = 128;
 
 // Lays the per-call buffers out in the context scratch; returns bytes needed
 // (base == nullptr only measures).
@@ -2062,77 +2119,19 @@ int launch_group(k3x_hip_ctx* ctx, const uint32_t* ids, uint32_t T, uint32_t K, 
     return launched(ctx, 3);
 }
 
-template <bool FP4, bool GATEUP, int MT, int NT>
-void launch_gemm(k3x_hip_ctx* ctx, GemmArgs& g, uint32_t experts_in_grid, uint32_t rows,
-                 hipStream_t stream = nullptr) {
+template <bool GATEUP, int MT, int NT>
+void launch_gemm(k3x_hip_ctx* ctx, GemmArgs& g, uint32_t experts_in_grid, uint32_t rows) {
     g.blocks_per_expert = rows / 16 / (4 * NT);
     const dim3 grid(experts_in_grid * g.blocks_per_expert);
-    if (!stream) stream = ctx->stream;
     if (g.a_lo)
-        hipLaunchKernelGGL((expert_gemm<FP4, GATEUP, MT, NT, true>), grid, dim3(256), 0, stream,
-                           g);
+        hipLaunchKernelGGL((expert_gemm<GATEUP, MT, NT, true>), grid, dim3(256), 0, ctx->stream, g);
     else
-        hipLaunchKernelGGL((expert_gemm<FP4, GATEUP, MT, NT, false>), grid, dim3(256), 0, stream,
+        hipLaunchKernelGGL((expert_gemm<GATEUP, MT, NT, false>), grid, dim3(256), 0, ctx->stream,
                            g);
-}
-
-// The shared expert below the wide GEMM's row counts: gate/up + GLU -> sact,
-// down -> sy, each as one block of T rows on the narrow GEMM, on `stream`
-// (stage marks only on the context stream).
-int run_shared_narrow(k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_hip_moe_params* p,
-                      const Scratch& s, const uint16_t* xn, const GluParams& glu, bool split_in,
-                      hipStream_t stream) {
-    const auto& d = bank->desc;
-    const uint32_t T = p->tokens;
-    const bool wide = T > 16;  // more than one 16-row MFMA tile
-    const bool marks = stream == ctx->stream;
-    GemmArgs sg{};
-    sg.status = ctx->status;
-    sg.glu = glu;
-    sg.top_k = p->top_k;
-    sg.codes = bank->sh_gu;
-    sg.kt = bank->sgate.kt;
-    sg.a = xn;
-    sg.a_stride = split_in ? 2 * d.hidden : d.hidden;
-    sg.a_lo = split_in ? d.hidden : 0;
-    sg.tokens = T;
-    sg.act = s.sact;
-    sg.act_stride = d.shared_inter;
-    sg.act_lo = 0;  // the bank's shared expert keeps bf16 activations
-    int mark = marks ? begin_stage(ctx, K3X_STAGE_SHARED_GATE_UP) : -1;
-    if (wide) launch_gemm<false, true, 4, 1>(ctx, sg, 1, d.shared_inter, stream);
-    else launch_gemm<false, true, 1, 1>(ctx, sg, 1, d.shared_inter, stream);
-    if (marks) end_stage(ctx, mark);
-    GemmArgs sd = sg;
-    sd.codes = bank->sh_dn;
-    sd.kt = bank->sdown.kt;
-    sd.a = s.sact;
-    sd.a_stride = d.shared_inter;
-    sd.a_lo = 0;
-    sd.y = s.sy;
-    sd.y_stride = d.hidden;
-    sd.scatter = 0;
-    mark = marks ? begin_stage(ctx, K3X_STAGE_SHARED_DOWN) : -1;
-    if (wide) launch_gemm<false, false, 4, 2>(ctx, sd, 1, d.hidden, stream);
-    else launch_gemm<false, false, 1, 2>(ctx, sd, 1, d.hidden, stream);
-    if (marks) end_stage(ctx, mark);
-    return launched(ctx, 2);
-}
-
-// The shared expert on the wide GEMM: output rows a multiple of the
-// workgroup's row blocks, K extents whole pipeline blocks.
-bool wide_shared_ok(const k3x_hip_layer_desc& d, uint32_t T) {
-    using k3x_hip::wide_rb_per_block;
-    constexpr uint32_t kq = 128 * k3x_hip::kWideStages;
-    return T >= kWideMinTokens && d.hidden % kq == 0 && d.shared_inter % kq == 0 &&
-           (d.shared_inter / 16) % wide_rb_per_block(k3x_hip::kWideSharedGateUp) == 0 &&
-           (d.hidden / 16) % wide_rb_per_block(k3x_hip::kWideSharedDown) == 0 &&
-           (uint64_t)T * std::max(d.hidden, d.shared_inter) * 2 < (1ull << 32) &&
-           (uint64_t)d.shared_inter * d.hidden * 4 < (1ull << 32);
 }
 
 // Many rows per expert: the wide grouped GEMM (128-row chunks, activations
-// staged in LDS) for the routed and the shared expert.  Shapes it needs: K
+// staged in LDS) for the routed experts.  Shapes it needs: K
 // tile counts even, output rows a multiple of the workgroup's row blocks,
 // element offsets of the activation rows below 2^32.
 bool use_wide_gemm(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, bool split) {
@@ -2143,7 +2142,6 @@ bool use_wide_gemm(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, bool spl
     return T >= kWideMinTokens && d.hidden % kq == 0 && d.inter % kq == 0 &&
            (d.inter / 16) % wide_rb_per_block(k3x_hip::kWideRoutedGateUp) == 0 &&
            (d.hidden / 16) % wide_rb_per_block(k3x_hip::kWideRoutedDown) == 0 &&
-           (!d.shared_inter || wide_shared_ok(d, T)) &&
            rows * std::max(d.hidden, d.inter * (split ? 2 : 1)) * 2 < (1ull << 32) &&
            // weight byte offsets within one matrix pair are 32-bit as well
            (uint64_t)d.inter * d.hidden * 4 < (1ull << 32);
@@ -2215,45 +2213,22 @@ k3x_hip::WideGemmArgs wide_gate_up_args(k3x_hip_ctx* ctx, const k3x_hip_bank* ba
     return g;
 }
 
-// The shared expert on the wide GEMM: gate/up + GLU -> sact, down -> sy, on
-// `stream` (stage marks only on the context stream).
-int run_shared_wide(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
-                    const Scratch& s, const uint16_t* xn, const GluParams& glu,
-                    hipStream_t stream) {
-    using namespace k3x_hip;
+// The shared expert: gate/up + GLU -> sact, down -> sy, on `stream` (stage
+// marks only on the context stream).  It keeps bf16 activations.
+int run_shared(k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_hip_moe_params* p,
+               const Scratch& s, const uint16_t* xn, const GluParams& glu, hipStream_t stream) {
     const auto& d = bank->desc;
     const uint32_t T = p->tokens;
-    const uint32_t all_chunks = (T + kWideRows - 1) / kWideRows;
     const bool marks = stream == ctx->stream;
-    WideGemmArgs sg = wide_gate_up_args(ctx, bank, p, s, xn, glu);
-    sg.codes = bank->sh_gu;
-    sg.scales = nullptr;
-    sg.codes_per_expert = 0;
-    sg.kt = bank->sgate.kt;
-    sg.nrb = d.shared_inter / 16;
-    sg.gather = 0;
-    sg.items = nullptr;
-    sg.tokens = T;
-    sg.act = s.sact;
-    sg.act_stride = d.shared_inter;
-    sg.act_lo = 0;  // the bank's shared expert keeps bf16 activations
     int mark = marks ? begin_stage(ctx, K3X_STAGE_SHARED_GATE_UP) : -1;
-    int st = launch_wide_gemm(ctx, kWideSharedGateUp, sg, all_chunks, stream);
+    int st = k3x_hip::dense_gate_up(ctx, reinterpret_cast<const uint4*>(bank->sh_gu),
+                                    d.shared_inter, d.hidden, xn, T, glu, s.sact, stream, false,
+                                    (p->flags & K3X_FLAG_SPLIT_INPUT) != 0);
     end_stage(ctx, mark);
     if (st) return st;
-    WideGemmArgs sd = sg;
-    sd.codes = bank->sh_dn;
-    sd.kt = bank->sdown.kt;
-    sd.nrb = d.hidden / 16;
-    sd.a = s.sact;
-    sd.a_stride = d.shared_inter;
-    sd.a_bytes = T * d.shared_inter * 2;
-    sd.act = nullptr;
-    sd.y = s.sy;
-    sd.y_stride = d.hidden;
-    sd.scatter = 0;
     mark = marks ? begin_stage(ctx, K3X_STAGE_SHARED_DOWN) : -1;
-    st = launch_wide_gemm(ctx, kWideSharedDown, sd, all_chunks, stream);
+    st = k3x_hip::dense_down(ctx, reinterpret_cast<const uint4*>(bank->sh_dn), d.hidden,
+                             d.shared_inter, s.sact, T, s.sy, stream);
     end_stage(ctx, mark);
     return st;
 }
@@ -2332,7 +2307,7 @@ int run_wide(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     end_stage(ctx, mark);
     if (st) return st;
     if (shared_inline && d.shared_inter &&
-        (st = run_shared_wide(ctx, bank, p, s, xn, glu, ctx->stream)))
+        (st = run_shared(ctx, bank, p, s, xn, glu, ctx->stream)))
         return st;
     WideGemmArgs dn = g;
     dn.codes = bank->dn_codes;
@@ -2364,15 +2339,6 @@ int run_wide(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     end_stage(ctx, mark);
     const int jst = cjoin.join();
     return st ? st : jst;
-}
-
-// The shared expert on `stream` (stage marks only on the context stream).
-int run_shared(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
-               const Scratch& s, const uint16_t* xn, const GluParams& glu, hipStream_t stream) {
-    const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
-    return !split_in && wide_shared_ok(bank->desc, p->tokens)
-               ? run_shared_wide(ctx, bank, p, s, xn, glu, stream)
-               : run_shared_narrow(ctx, bank, p, s, xn, glu, split_in, stream);
 }
 
 // Grouping, expert GEMMs, shared expert, combine.  xn is the bf16 input of
@@ -2560,7 +2526,7 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     if (few) {
         if ((st = k3x_hip::launch_few_row_gate_up(ctx, bank, T, K, s, xn, glu, split))) return st;
     } else {
-        launch_gemm<true, true, 4, 1>(ctx, g, max_active, d.inter);
+        launch_gemm<true, 4, 1>(ctx, g, max_active, d.inter);
     }
     end_stage(ctx, mark);
     // Routed down, scattered to [token][slot].
@@ -2577,7 +2543,6 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     dn.gather = 0;
     dn.y = s.y;
     dn.y_stride = d.hidden;
-    dn.scatter = 1;
     // Few tokens: the combine rides in the down launch (the decode path's
     // fused mix), after the shared expert, whose output it adds.
     if (few && k3x_hip::few_row_mix_eligible(bank, T)) {
@@ -2596,7 +2561,7 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     if (few) {
         if ((st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split))) return st;
     } else {
-        launch_gemm<true, false, 4, 2>(ctx, dn, max_active, d.hidden);
+        launch_gemm<false, 4, 2>(ctx, dn, max_active, d.hidden);
     }
     end_stage(ctx, mark);
     if ((st = launched(ctx, few ? 0 : 2))) return st;
@@ -2870,11 +2835,34 @@ int launch_topk(k3x_hip_ctx* ctx, const float* logits, const float* bias, uint32
 // Dense bf16 projections in the bank's tile layout: the wide grouped GEMM
 // (one item per 128-row chunk of the T rows) from kWideMinTokens rows when
 // the shapes fit it, else expert_gemm over the T rows as one block.
+// The wide GEMM's dense kinds: shapes, and the tokens from which they beat
+// the rows kernel.
+bool dense_wide_ok(WideKind kind, uint32_t N, uint32_t K, uint32_t T) {
+    return T >= kDenseWideTokens && K % (128 * kWideStages) == 0 &&
+           (N / 16) % wide_rb_per_block(kind) == 0 && N % 16 == 0 &&
+           (uint64_t)T * std::max(N, K) * 4 < (1ull << 32) && (uint64_t)N * K * 4 < (1ull << 32);
+}
+
+template <int S, int OUT, bool SPLIT>
+int launch_dense_rows(k3x_hip_ctx* ctx, const GemvArgs& g, uint32_t N, hipStream_t stream) {
+    if (g.tokens <= 32) {
+        hipLaunchKernelGGL((dense_rows_kernel<S, 1, 2, OUT, SPLIT>), dim3(N / 16),
+                           dim3(64 * kRowsWaves), 0, stream, g);
+    } else {
+        constexpr int NB = 3 - S;  // N % 32 == 0 (checked by the callers)
+        hipLaunchKernelGGL((dense_rows_kernel<S, NB, 4, OUT, SPLIT>),
+                           dim3(N / 16 / NB, (g.tokens + 63) / 64), dim3(64 * kRowsWaves), 0,
+                           stream, g);
+    }
+    return launched(ctx, 1);
+}
+
 int dense_down_output(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K,
                       const uint16_t* a, uint32_t T, const float* prefix, const float* shared,
                       float* routed, uint16_t* out) {
-    if (!T || T > kGemvMaxTokens || N % 128 || K % 128) return K3X_ERR_INVALID_EXTENT;
+    if (!T || N % 128 || K % 128) return K3X_ERR_INVALID_EXTENT;
     GemvArgs g{tiles, K / 128, a, K, T, out, N, {}, ctx->status, prefix, shared, routed};
+    if (T > kGemvMaxTokens) return launch_dense_rows<1, 3, false>(ctx, g, N, ctx->stream);
     if (K / 128 <= 2 * kGemvWaves && (size_t)T * K / 8 <= 64 * kGemvWaves &&
         (uintptr_t)a % 16 == 0)
         hipLaunchKernelGGL((dense_gemv_kernel<1, 2, 3, kGemvWaves, false, true>), dim3(N / 16),
@@ -2904,27 +2892,16 @@ int dense_norm_output(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t
     return launched(ctx, 1);
 }
 
-bool dense_wide_ok(WideKind kind, uint32_t N, uint32_t K, uint32_t T) {
-    return T >= kWideMinTokens && K % (128 * kWideStages) == 0 &&
-           (N / 16) % wide_rb_per_block(kind) == 0 && N % 16 == 0 &&
-           (uint64_t)T * std::max(N, K) * 4 < (1ull << 32) && (uint64_t)N * K * 4 < (1ull << 32);
-}
-
-bool dense_mlp_any_stream(uint32_t I, uint32_t H, uint32_t T) {
-    return T <= kDenseDirectTokens ||
-           (dense_wide_ok(kWideSharedGateUp, I, H, T) && dense_wide_ok(kWideSharedDown, H, I, T));
-}
-
-bool dense_down_any_stream(uint32_t N, uint32_t K, uint32_t T) {
-    return T <= kDenseDirectTokens || dense_wide_ok(kWideSharedDown, N, K, T);
+bool dense_direct(uint32_t N, uint32_t K, uint32_t T) {
+    return !dense_wide_ok(kWideSharedDown, N, K, T);
 }
 
 int dense_gate_up(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t I, uint32_t H, const uint16_t* x,
                   uint32_t T, const GluParams& glu, uint16_t* act, hipStream_t stream,
-                  bool split) {
+                  bool split, bool split_in) {
     if (!T || I % 64 || H % 128) return K3X_ERR_INVALID_EXTENT;
     const uint32_t act_stride = split ? 2 * I : I, act_lo = split ? I : 0;
-    if (dense_wide_ok(kWideSharedGateUp, I, H, T)) {
+    if (!split_in && dense_wide_ok(kWideSharedGateUp, I, H, T)) {
         WideGemmArgs g{};
         g.codes = reinterpret_cast<const uint8_t*>(tiles);
         g.kt = H / 128;
@@ -2940,9 +2917,10 @@ int dense_gate_up(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t I, uint32_t H, 
         g.status = ctx->status;
         return launch_wide_gemm(ctx, kWideSharedGateUp, g, (T + kWideRows - 1) / kWideRows, stream);
     }
-    if (T <= kGemvMaxTokens) {
-        GemvArgs g{tiles, H / 128, x, H, T, act, act_stride, glu, ctx->status};
-        g.out_lo = act_lo;
+    GemvArgs g{tiles, H / 128, x, split_in ? 2 * H : H, T, act, act_stride, glu, ctx->status};
+    g.out_lo = act_lo;
+    g.x_lo = split_in ? H : 0;
+    if (T <= kGemvMaxTokens && !split_in) {
         // Beside the context stream: half-size workgroups, so that the
         // other stream's launches find room on every compute unit.
         if (stream == ctx->stream)
@@ -2953,21 +2931,8 @@ int dense_gate_up(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t I, uint32_t H, 
                                dim3(32 * kGemvWaves), 0, stream, g);
         return launched(ctx, 1);
     }
-    if (stream != ctx->stream) return K3X_ERR_INVALID_EXTENT;
-    GemmArgs g{};
-    g.codes = reinterpret_cast<const uint8_t*>(tiles);
-    g.kt = H / 128;
-    g.a = x;
-    g.a_stride = H;
-    g.tokens = T;
-    g.act = act;
-    g.act_stride = act_stride;
-    g.act_lo = act_lo;
-    g.glu = glu;
-    g.status = ctx->status;
-    if (T > 16) launch_gemm<false, true, 4, 1>(ctx, g, 1, I);
-    else launch_gemm<false, true, 1, 1>(ctx, g, 1, I);
-    return launched(ctx, 1);
+    return split_in ? launch_dense_rows<2, 2, true>(ctx, g, I, stream)
+                    : launch_dense_rows<2, 2, false>(ctx, g, I, stream);
 }
 
 int dense_down(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K, const uint16_t* a,
@@ -2975,12 +2940,27 @@ int dense_down(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K, con
     if (!T || N % 128 || K % 128) return K3X_ERR_INVALID_EXTENT;
     // Split rows [hi | lo] of 2 K: each weight tile meets both halves.
     const uint32_t a_stride = split ? 2 * K : K;
+    if (y_bf16 && (split || !dense_direct(N, K, T))) return K3X_ERR_INVALID_EXTENT;
+    if (!dense_direct(N, K, T)) {
+        WideGemmArgs g{};
+        g.codes = reinterpret_cast<const uint8_t*>(tiles);
+        g.kt = K / 128;
+        g.kta = split ? 2 * g.kt : 0;  // the weights repeated along K
+        g.nrb = N / 16;
+        g.a = a;
+        g.a_stride = a_stride;
+        g.a_bytes = T * a_stride * 2;
+        g.tokens = T;
+        g.y = y;
+        g.y_stride = N;
+        g.status = ctx->status;
+        return launch_wide_gemm(ctx, kWideSharedDown, g, (T + kWideRows - 1) / kWideRows, stream);
+    }
+    GemvArgs g{tiles, K / 128, a, a_stride, T, y_bf16 ? (void*)y_bf16 : (void*)y, N, {},
+               ctx->status};
+    g.x_lo = split ? K : 0;
     if (T <= kGemvMaxTokens) {
-        GemvArgs g{tiles, K / 128, a, a_stride, T, y_bf16 ? (void*)y_bf16 : (void*)y, N, {},
-                   ctx->status};
-        g.x_lo = split ? K : 0;
         const dim3 grid(N / 16);
-        if (y_bf16 && split) return K3X_ERR_INVALID_EXTENT;
         if (y_bf16)
             hipLaunchKernelGGL((dense_gemv_kernel<1, 3, 1>), grid, dim3(64 * kGemvWaves), 0, stream,
                                g);
@@ -2998,36 +2978,9 @@ int dense_down(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K, con
                                dim3(32 * kGemvWaves), 0, stream, g);
         return launched(ctx, 1);
     }
-    if (y_bf16) return K3X_ERR_INVALID_EXTENT;
-    if (dense_wide_ok(kWideSharedDown, N, K, T)) {
-        WideGemmArgs g{};
-        g.codes = reinterpret_cast<const uint8_t*>(tiles);
-        g.kt = K / 128;
-        g.kta = split ? 2 * g.kt : 0;  // the weights repeated along K
-        g.nrb = N / 16;
-        g.a = a;
-        g.a_stride = a_stride;
-        g.a_bytes = T * a_stride * 2;
-        g.tokens = T;
-        g.y = y;
-        g.y_stride = N;
-        g.status = ctx->status;
-        return launch_wide_gemm(ctx, kWideSharedDown, g, (T + kWideRows - 1) / kWideRows, stream);
-    }
-    if (stream != ctx->stream) return K3X_ERR_INVALID_EXTENT;
-    GemmArgs g{};
-    g.codes = reinterpret_cast<const uint8_t*>(tiles);
-    g.kt = K / 128;
-    g.a_lo = split ? K : 0;
-    g.a = a;
-    g.a_stride = a_stride;
-    g.tokens = T;
-    g.y = y;
-    g.y_stride = N;
-    g.status = ctx->status;
-    if (T > 16) launch_gemm<false, false, 4, 2>(ctx, g, 1, N);
-    else launch_gemm<false, false, 1, 2>(ctx, g, 1, N);
-    return launched(ctx, 1);
+    if (y_bf16) return launch_dense_rows<1, 1, false>(ctx, g, N, stream);
+    return split ? launch_dense_rows<1, 0, true>(ctx, g, N, stream)
+                 : launch_dense_rows<1, 0, false>(ctx, g, N, stream);
 }
 
 size_t router_wp_floats(uint32_t experts) {
