@@ -688,7 +688,10 @@ __global__ __launch_bounds__(64) void topk_reg_kernel(const float* __restrict__ 
 //   renorm     one wave, sequential sums in slot order, as topk_wave.
 // Same results as topk_reg_kernel, bit for bit.
 constexpr uint32_t kTopkThrThreads = 256;
-constexpr uint32_t kTopkThrMaxTokens = 256;  // tokens up to which launch_topk_any uses it
+// Tokens up to which launch_topk_any uses it for 256 < E <= 512 (beyond, the
+// wave kernel is level with it); above 512 experts it always does (896
+// experts, 2048 tokens, router and Top-K: 412 -> 395 us).
+constexpr uint32_t kTopkThrMaxTokens = 256;
 
 // PUBLISH: ids and weights are stored at device scope (coherent across the
 // XCDs' L2s), for a workgroup of the same launch to read them.
@@ -1872,6 +1875,12 @@ int launched(k3x_hip_ctx* ctx, unsigned n) {
 // the decode kernels, {expert, rows, CSR offset, tokens of the first four
 // rows (8 bits each)}, in active_asc order.
 constexpr uint32_t kGroupSmallPairs = 256;
+// Tokens up to which routes are grouped so (and with their Top-K in one
+// launch): its passes over the pairs are serial, so past the few-token calls
+// the chunked kernels are shorter (Top-K and grouping of 13 tokens, 384
+// experts, Top-16, with the router's 20 us: 72 us in one launch, 40 in two).
+constexpr uint32_t kGroupSmallTokens = 4;
+static_assert(kGroupSmallTokens * 64 <= kGroupSmallPairs, "top_k is at most 64");
 static_assert(kGroupSmallPairs == kTopkThrThreads, "the fused Top-K launch groups with its threads");
 
 // ATOMIC: the ids are read at device scope (written in the same launch by
@@ -2095,7 +2104,7 @@ int launch_group(k3x_hip_ctx* ctx, const uint32_t* ids, uint32_t T, uint32_t K, 
     uint32_t* chunk_fu = chunk_cnt + (size_t)nch * E;
     uint8_t* rank = reinterpret_cast<uint8_t*>(chunk_fu + (size_t)nch * E);
     const uint32_t chunk_rows = srec ? srec_rows : k3x_hip::kWideRows;
-    if (!witems && T * K <= kGroupSmallPairs) {
+    if (!witems && T <= kGroupSmallTokens) {
         hipLaunchKernelGGL(group_small_kernel, dim3(1), dim3(kGroupSmallPairs), 0, ctx->stream,
                            ids, T, K, E, ready, counts, offsets, first_use, n_active, active_asc,
                            active_fu, pair_token, pair_slot, arec, ctx->status);
@@ -2168,7 +2177,7 @@ RoutedKind routed_kind(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank,
     const uint32_t T = p->tokens, K = p->top_k;
     const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
     const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
-    if (!split_in && T * K <= kGroupSmallPairs &&
+    if (!split_in && T <= kGroupSmallTokens &&
         k3x_hip::few_row_experts_eligible(ctx, bank, T, split))
         return kRoutedFew;
     if (!split_in && T >= (scaled_fp4(p) ? kWideMinTokens : kStreamMaxTokens) &&
@@ -2414,7 +2423,7 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     // The wide GEMM takes work items, the streaming one records: row chunks
     // (srec), or one an active expert from the small-route grouping (arec;
     // the decode path's kernels read the same records).
-    const bool small = kind != kRoutedWide && T * K <= kGroupSmallPairs;
+    const bool small = kind != kRoutedWide && T <= kGroupSmallTokens;
     const bool chunks = kind == kRoutedStream && !small;
     const uint32_t srec_rows = stream_record_rows(d, T, K);
     uint2* const srec = reinterpret_cast<uint2*>(s.arec);
@@ -2678,11 +2687,10 @@ int launch_topk_any(k3x_hip_ctx* ctx, const float* logits, const float* bias, ui
     hipLaunchKernelGGL(topk_thr_kernel<ept>, dim3(T), dim3(kTopkThrThreads), 0, ctx->stream,    \
                        logits, bias, E, K, routed_scale, renorm, ids, weights, ctx->status)
     if (T <= kTopkThrMaxTokens && E > 256 && E <= 512) K3X_TOPK_THR(2);
-    else if (T <= kTopkThrMaxTokens && E > 512 && E <= 1024) K3X_TOPK_THR(4);
+    else if (E > 512 && E <= 1024) K3X_TOPK_THR(4);
 #undef K3X_TOPK_THR
     else if (E <= 256) K3X_TOPK(4);
     else if (E <= 512) K3X_TOPK(8);
-    else if (E <= 1024) K3X_TOPK(16);
 #undef K3X_TOPK
     else
         hipLaunchKernelGGL(topk_kernel, dim3(T), dim3(64), (size_t)E * 12, ctx->stream, logits,
@@ -2795,8 +2803,7 @@ int launch_official_select(k3x_hip_ctx* ctx, const OfficialDecode& d, const Laye
 }
 
 bool topk_group_eligible(uint32_t E, uint32_t K, uint32_t T) {
-    return E > 256 && E <= 1024 && T >= 1 && T <= kTopkThrMaxTokens && K >= 1 && K <= 64 &&
-           (size_t)T * K <= kGroupSmallPairs && T < kWideMinTokens;
+    return E > 256 && E <= 1024 && T >= 1 && T <= kGroupSmallTokens && K >= 1 && K <= 64;
 }
 
 int launch_topk_group(k3x_hip_ctx* ctx, const float* logits, const float* bias, uint32_t E,
