@@ -24,13 +24,11 @@ inline unsigned blocks_for(size_t n) { return (unsigned)((n + kThreads - 1) / kT
 // memory (src != nullptr) or the seeded generator (src == nullptr, key).
 // ---------------------------------------------------------------------------
 
-// MXFP4 codes -> tiles [rb][kt][S][64] x 16 B (S = 2 for interleaved gate/up).
-__global__ void retile_fp4_codes(const uint8_t* __restrict__ src, uint64_t key,
-                                 uint32_t rows, uint32_t cols, uint32_t kt,
-                                 uint32_t S, uint32_t which, uint4* __restrict__ dst) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t total = (size_t)(rows / 16) * kt * 64;
-    if (t >= total) return;
+// MXFP4 codes -> tiles [rb][kt][S][64] x 16 B (S = 2 for interleaved
+// gate/up): word t of the matrix.
+__device__ inline void retile_fp4_codes(const uint8_t* __restrict__ src, uint64_t key, size_t t,
+                                        uint32_t cols, uint32_t kt, uint32_t S, uint32_t which,
+                                        uint4* __restrict__ dst) {
     const uint32_t lane = t % 64;
     const uint32_t k = (uint32_t)((t / 64) % kt);
     const size_t rb = t / (64 * (size_t)kt);
@@ -48,14 +46,12 @@ __global__ void retile_fp4_codes(const uint8_t* __restrict__ src, uint64_t key,
     dst[((rb * kt + k) * S + which) * 64 + lane] = v;
 }
 
-// E8M0 scales -> dwords [rb][ks][S][64]; byte b of a dword is K-tile 4q+b.
-__global__ void retile_fp4_scales(const uint8_t* __restrict__ src, uint64_t key,
-                                  uint32_t lo, uint32_t span, uint32_t rows,
-                                  uint32_t cols, uint32_t kt, uint32_t ks, uint32_t S,
-                                  uint32_t which, uint32_t* __restrict__ dst) {
-    const size_t t = (size_t)blockIdx.x * blockDim.x + threadIdx.x;
-    const size_t total = (size_t)(rows / 16) * ks * 64;
-    if (t >= total) return;
+// E8M0 scales -> dwords [rb][ks][S][64]; byte b of a dword is K-tile 4q+b:
+// dword t of the matrix.
+__device__ inline void retile_fp4_scales(const uint8_t* __restrict__ src, uint64_t key, size_t t,
+                                         uint32_t lo, uint32_t span, uint32_t cols, uint32_t kt,
+                                         uint32_t ks, uint32_t S, uint32_t which,
+                                         uint32_t* __restrict__ dst) {
     const uint32_t lane = t % 64;
     const uint32_t q = (uint32_t)((t / 64) % ks);
     const size_t rb = t / (64 * (size_t)ks);
@@ -73,6 +69,45 @@ __global__ void retile_fp4_scales(const uint8_t* __restrict__ src, uint64_t key,
         packed |= s << (8 * b);
     }
     dst[((rb * ks + q) * S + which) * 64 + lane] = packed;
+}
+
+// One expert's six arrays in one launch: workgroups [first[i], first[i + 1])
+// re-tile array i (gate codes, gate scales, up codes, up scales, down codes,
+// down scales).  check: the extents' results of the launch before; the slot
+// is written, and marked admitted, only if every CRC is the expected one
+// (expect null: not asked) and no scale byte is 0xFF.
+struct RetileArgs {
+    const uint8_t* src[6];
+    uint64_t key[6];
+    uint32_t first[7];
+    uint32_t lo, span;
+    uint32_t rows[2], cols[2], kt[2], ks[2];  // gate and up, down
+    uint4* codes[2];
+    uint32_t* scales[2];
+    const k3x_hip::ExtentResult* check;
+    uint32_t expect[6];
+    uint32_t use_crc;
+    uint32_t* ready;  // the slot's admitted word, or null
+};
+
+__global__ __launch_bounds__(kThreads) void retile_expert_kernel(RetileArgs a) {
+    if (a.check) {
+        for (uint32_t i = 0; i < 6; ++i)
+            if ((a.use_crc && a.check->raw[i] != a.expect[i]) || (i % 2 && a.check->ff[i])) return;
+    }
+    uint32_t i = 0;
+    while (blockIdx.x >= a.first[i + 1]) ++i;
+    const uint32_t d = i / 4, S = d ? 1u : 2u, which = d ? 0u : i / 2;
+    const size_t t = (size_t)(blockIdx.x - a.first[i]) * kThreads + threadIdx.x;
+    const size_t per = (size_t)(a.rows[d] / 16) * 64;
+    if (i % 2) {
+        if (t < per * a.ks[d])
+            retile_fp4_scales(a.src[i], a.key[i], t, a.lo, a.span, a.cols[d], a.kt[d], a.ks[d], S,
+                              which, a.scales[d]);
+    } else if (t < per * a.kt[d]) {
+        retile_fp4_codes(a.src[i], a.key[i], t, a.cols[d], a.kt[d], S, which, a.codes[d]);
+    }
+    if (a.ready && blockIdx.x == 0 && threadIdx.x == 0) *a.ready = 1u;
 }
 
 // bf16 matrix -> tiles [rb][kt][S][4][64] x 16 B (8 bf16 per lane per MFMA).
@@ -209,39 +244,45 @@ int alloc(T** p, size_t bytes, uint64_t* total) {
     return K3X_OK;
 }
 
-// Launches the four re-tile kernels of one routed expert.
-int retile_expert(k3x_hip_bank* b, uint32_t e, const uint8_t* src[6], uint64_t seed,
-                  uint32_t lo, uint32_t span) {
+// Re-tiles one routed expert into its slot (src null: from the generator).
+// expect: the extents' results are checked on the device first (use_crc: the
+// raw CRCs too) and the slot's admitted word is set.
+int retile_expert(k3x_hip_bank* b, uint32_t e, const uint8_t* const src[6], uint64_t seed,
+                  uint32_t lo, uint32_t span, const uint32_t* expect = nullptr,
+                  bool use_crc = false) {
     k3x_hip_ctx* ctx = b->ctx;
-    const MatrixGeom& G = b->gate;
-    const MatrixGeom& D = b->down;
-    uint4* gu = reinterpret_cast<uint4*>(b->gu_codes + e * b->gu_codes_per_expert);
-    uint32_t* gus = b->gu_scales + e * b->gu_scales_per_expert;
-    uint4* dn = reinterpret_cast<uint4*>(b->dn_codes + e * b->dn_codes_per_expert);
-    uint32_t* dns = b->dn_scales + e * b->dn_scales_per_expert;
-    const uint64_t ex = e;
-    auto key = [&](uint64_t kind) { return stream_key(seed, (kind << 32) | ex); };
-    const size_t gcodes = (size_t)(G.rows / 16) * G.kt * 64;
-    const size_t gscales = (size_t)(G.rows / 16) * G.ks * 64;
-    for (uint32_t which = 0; which < 2; ++which) {
-        const uint64_t ck = which ? K3X_STREAM_UP_CODES : K3X_STREAM_GATE_CODES;
-        const uint64_t sk = which ? K3X_STREAM_UP_SCALES : K3X_STREAM_GATE_SCALES;
-        hipLaunchKernelGGL(retile_fp4_codes, dim3(blocks_for(gcodes)), dim3(kThreads), 0,
-                           ctx->stream, src[2 * which], key(ck), G.rows, G.cols, G.kt, 2u,
-                           which, gu);
-        hipLaunchKernelGGL(retile_fp4_scales, dim3(blocks_for(gscales)), dim3(kThreads), 0,
-                           ctx->stream, src[2 * which + 1], key(sk), lo, span, G.rows, G.cols,
-                           G.kt, G.ks, 2u, which, gus);
+    const MatrixGeom* geom[2] = {&b->gate, &b->down};
+    constexpr uint64_t kind[6] = {K3X_STREAM_GATE_CODES, K3X_STREAM_GATE_SCALES,
+                                  K3X_STREAM_UP_CODES,   K3X_STREAM_UP_SCALES,
+                                  K3X_STREAM_DOWN_CODES, K3X_STREAM_DOWN_SCALES};
+    RetileArgs a{};
+    for (int d = 0; d < 2; ++d) {
+        a.rows[d] = geom[d]->rows;
+        a.cols[d] = geom[d]->cols;
+        a.kt[d] = geom[d]->kt;
+        a.ks[d] = geom[d]->ks;
     }
-    const size_t dcodes = (size_t)(D.rows / 16) * D.kt * 64;
-    const size_t dscales = (size_t)(D.rows / 16) * D.ks * 64;
-    hipLaunchKernelGGL(retile_fp4_codes, dim3(blocks_for(dcodes)), dim3(kThreads), 0,
-                       ctx->stream, src[4], key(K3X_STREAM_DOWN_CODES), D.rows, D.cols, D.kt,
-                       1u, 0u, dn);
-    hipLaunchKernelGGL(retile_fp4_scales, dim3(blocks_for(dscales)), dim3(kThreads), 0,
-                       ctx->stream, src[5], key(K3X_STREAM_DOWN_SCALES), lo, span, D.rows,
-                       D.cols, D.kt, D.ks, 1u, 0u, dns);
-    return check_launch(ctx, 6);
+    for (int i = 0; i < 6; ++i) {
+        const MatrixGeom& g = *geom[i / 4];
+        a.src[i] = src[i];
+        a.key[i] = stream_key(seed, (kind[i] << 32) | e);
+        a.first[i + 1] =
+            a.first[i] + blocks_for((size_t)(g.rows / 16) * 64 * (i % 2 ? g.ks : g.kt));
+    }
+    a.lo = lo;
+    a.span = span;
+    a.codes[0] = reinterpret_cast<uint4*>(b->gu_codes + e * b->gu_codes_per_expert);
+    a.codes[1] = reinterpret_cast<uint4*>(b->dn_codes + e * b->dn_codes_per_expert);
+    a.scales[0] = b->gu_scales + e * b->gu_scales_per_expert;
+    a.scales[1] = b->dn_scales + e * b->dn_scales_per_expert;
+    if (expect) {
+        a.check = &ctx->crc_state->result;
+        for (int i = 0; i < 6; ++i) a.expect[i] = expect[i];
+        a.use_crc = use_crc;
+        a.ready = b->ready_dev + e;
+    }
+    hipLaunchKernelGGL(retile_expert_kernel, dim3(a.first[6]), dim3(kThreads), 0, ctx->stream, a);
+    return check_launch(ctx);
 }
 
 int retile_shared(k3x_hip_bank* b, const uint16_t* src[3], uint64_t seed, float sigma) {
@@ -274,12 +315,6 @@ int set_expert_ready(k3x_hip_bank* b, uint32_t e, bool ready) {
                              b->ctx->stream) == hipSuccess
                ? K3X_OK
                : K3X_ERR_BACKEND_UNAVAILABLE;
-}
-
-int retile_expert_device(k3x_hip_bank* b, uint32_t e, const uint8_t* const src[6]) {
-    const uint8_t* s[6];
-    for (int i = 0; i < 6; ++i) s[i] = src[i];
-    return retile_expert(b, e, s, 0, 0, 1);
 }
 
 int retile_bf16_matrix(k3x_hip_ctx* ctx, const uint16_t* src, uint64_t key, float sigma,
@@ -694,29 +729,37 @@ int k3x_hip_bank_upload_expert_device(k3x_hip_bank* bank, uint32_t expert,
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
     const size_t n = (size_t)d.inter * d.hidden;
     const size_t len[6] = {n / 2, n / 32, n / 2, n / 32, n / 2, n / 32};
-    // Integrity and validity before the slot is touched.
-    for (int i = 0; i < 6; ++i) {
-        if (crc32c) {
-            uint32_t c = 0;
-            if (int st = k3x_hip::crc32c_device(ctx, extents[i], len[i], &c)) return st;
-            if (c != crc32c[i])
-                return i % 2 ? K3X_ERR_AUXILIARY_CRC_MISMATCH : K3X_ERR_DATA_CRC_MISMATCH;
-        }
-        if (i % 2) {
-            bool ff = false;
-            if (int st = k3x_hip::any_ff_device(ctx, extents[i], len[i], &ff)) return st;
-            if (ff) return K3X_ERR_INVALID_MXFP4;
-        }
+    // Integrity and validity are checked on the device before the slot is
+    // touched, in one launch over the extents (the codes only for their
+    // CRCs); the re-tile launch behind it reads the results and leaves the
+    // slot alone if any fails, so one wait serves both.
+    k3x_hip::Extent ext[6];
+    uint32_t n_ext = 0, expect[6] = {};
+    for (uint32_t i = 0; i < 6; ++i) {
+        if (crc32c) expect[i] = k3x_hip::raw_of_crc(crc32c[i], len[i]);
+        if (crc32c || i % 2) ext[n_ext++] = {extents[i], len[i], i, i % 2 != 0};
     }
-    int st = k3x_hip::set_expert_ready(bank, expert, false);
-    if (st) return st;
+    int st = k3x_hip::launch_extent_check(ctx, ext, n_ext);
+    st = st ? st : retile_expert(bank, expert, extents, 0, 0, 1, expect, crc32c != nullptr);
+    if (hipStreamSynchronize(ctx->stream) != hipSuccess) st = K3X_ERR_BACKEND_UNAVAILABLE;
+    if (!st)
+        for (int i = 0; i < 6; ++i) {
+            if (crc32c && ctx->crc_host->raw[i] != expect[i])
+                return i % 2 ? K3X_ERR_AUXILIARY_CRC_MISMATCH : K3X_ERR_DATA_CRC_MISMATCH;
+            if (i % 2 && ctx->crc_host->ff[i]) return K3X_ERR_INVALID_MXFP4;
+        }
+    // Whatever the slot held is no longer resident: its ids stop resolving to
+    // it, also if a device failure left it in an unknown state.
     for (auto it = bank->tensor_ids.begin(); it != bank->tensor_ids.end();)
         it = it->second / 4 == expert ? bank->tensor_ids.erase(it) : std::next(it);
-    st = k3x_hip::retile_expert_device(bank, expert, extents);
-    if (hipStreamSynchronize(ctx->stream) != hipSuccess) st = K3X_ERR_BACKEND_UNAVAILABLE;
-    if (st) return st;
+    bank->expert_ready[expert] = 0;
+    if (st) {
+        (void)k3x_hip::set_expert_ready(bank, expert, false);
+        return st;
+    }
     for (int m = 0; m < 3; ++m) bank->tensor_ids[tensor_ids[m]] = expert * 4 + (uint32_t)m;
-    return k3x_hip::set_expert_ready(bank, expert, true);
+    bank->expert_ready[expert] = 1;  // the device's word was set with the slot
+    return K3X_OK;
 }
 
 int k3x_hip_bank_find(k3x_hip_bank* bank, uint64_t tensor_id, uint32_t* expert, uint32_t* matrix) {

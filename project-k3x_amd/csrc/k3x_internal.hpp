@@ -18,6 +18,21 @@ struct StageMark {
     hipEvent_t stop;
 };
 
+namespace k3x_hip {
+// Extents of one CRC launch: an expert's six (gate, up and down codes and
+// scales, in the storage order).
+constexpr uint32_t kExtents = 6;
+struct ExtentResult {
+    uint32_t raw[kExtents];  // raw CRC32C
+    uint32_t ff[kExtents];   // a 0xFF byte was found
+};
+struct ExtentState {
+    uint32_t counts[kExtents];  // chunks done; zero between launches
+    uint32_t hits[kExtents];    // 0xFF found; zero between launches
+    ExtentResult result;
+};
+}  // namespace k3x_hip
+
 struct k3x_hip_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
@@ -57,8 +72,11 @@ struct k3x_hip_ctx {
     std::vector<hipEvent_t> free_events;
     double stage_ms[K3X_STAGE_COUNT] = {};
     uint64_t stage_launches[K3X_STAGE_COUNT] = {};
-    // CRC32C: device tables (uploaded at first use), chunk results, flag.
+    // CRC32C: device tables (uploaded at first use) with the extent state
+    // behind them, pinned results, chunk values.
     uint32_t* crc_tables = nullptr;
+    k3x_hip::ExtentState* crc_state = nullptr;
+    k3x_hip::ExtentResult* crc_host = nullptr;
     uint32_t* crc_chunks = nullptr;
     size_t crc_chunk_cap = 0;
 };
@@ -278,10 +296,20 @@ int dense_norm_output(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t
 
 // CRC32C of device bytes (storage.hip); *crc the standard value.
 int crc32c_device(k3x_hip_ctx* ctx, const void* data, size_t bytes, uint32_t* crc);
-// Whether any of `bytes` device bytes is 0xFF (MXFP4 scale validity).
-int any_ff_device(k3x_hip_ctx* ctx, const void* data, size_t bytes, bool* found);
+// One launch over up to kExtents device extents (16-byte aligned, multiples
+// of 16 bytes): each one's raw CRC32C (from a zero register) and, with
+// find_ff, whether any byte is 0xFF, to words `slot` of ctx->crc_state's
+// result on the device and of ctx->crc_host once the stream has passed.
+struct Extent {
+    const void* data;
+    uint64_t bytes;
+    uint32_t slot;
+    bool find_ff;
+};
+int launch_extent_check(k3x_hip_ctx* ctx, const Extent* ext, uint32_t n);
+// The raw CRC32C of `bytes` bytes whose standard CRC32C is crc.
+uint32_t raw_of_crc(uint32_t crc, uint64_t bytes);
 void free_crc(k3x_hip_ctx* ctx);
-int retile_expert_device(k3x_hip_bank* b, uint32_t e, const uint8_t* const src[6]);
 // Marks slot e admitted (1) or not (0) on the host and, in stream order, on
 // the device.
 int set_expert_ready(k3x_hip_bank* b, uint32_t e, bool ready);
