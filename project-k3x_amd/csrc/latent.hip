@@ -43,7 +43,7 @@ __device__ inline float situ(float g, float u, float beta, int has_linear, float
 }
 
 // One output row per wave, T <= kMaxTokens tokens per pass (x rows
-// [T][x_stride]); VEC: 16-byte loads (cols % 4 == 0, rows 16-byte aligned).
+// [T][x_stride]): shapes that the vector kernel below does not take.
 // OUT: 0 y = Wx; 1 y = Wx + add (fp32 add, as routed[row] += shared[row]);
 // 2 y = Wx and the split copy ys = [bf16 hi | bf16 lo] rows of 2 rows_total;
 // 3 y = situ(W x, W2 x) (the gate / up pair of an MLP).
@@ -63,7 +63,7 @@ struct GemvArgs {
     const uint32_t* status;
 };
 
-template <int OUT, bool VEC>
+template <int OUT>
 __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
     if (*(volatile const uint32_t*)a.status) return;
     const uint32_t lane = threadIdx.x & 63;
@@ -80,51 +80,16 @@ __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
         for (int m = 0; m < M; ++m)
 #pragma unroll
             for (uint32_t t = 0; t < kMaxTokens; ++t) acc[m][t] = 0.0;
-        if constexpr (VEC) {
-            // Four 16-byte loads per lane in flight (4 KiB per wave).
-            constexpr uint32_t kStep = 64 * 4 * 4;
-            for (uint32_t c0 = 0; c0 < a.cols; c0 += kStep) {
-                float4 w[M][4];
+        for (uint32_t c = lane; c < a.cols; c += 64) {
+            float w[M];
 #pragma unroll
-                for (int m = 0; m < M; ++m)
+            for (int m = 0; m < M; ++m) w[m] = wr[m][c];
 #pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint32_t c = c0 + (q * 64 + lane) * 4;
-                        w[m][q] = c < a.cols ? *reinterpret_cast<const float4*>(wr[m] + c)
-                                             : make_float4(0.f, 0.f, 0.f, 0.f);
-                    }
+            for (uint32_t t = 0; t < kMaxTokens; ++t) {
+                if (t >= nt) break;
+                const double xv = (double)a.x[(size_t)(t0 + t) * a.x_stride + c];
 #pragma unroll
-                for (uint32_t t = 0; t < kMaxTokens; ++t) {
-                    if (t >= nt) break;
-                    const float* xr = a.x + (size_t)(t0 + t) * a.x_stride;
-#pragma unroll
-                    for (int q = 0; q < 4; ++q) {
-                        const uint32_t c = c0 + (q * 64 + lane) * 4;
-                        if (c >= a.cols) continue;
-                        const float4 xv = *reinterpret_cast<const float4*>(xr + c);
-#pragma unroll
-                        for (int m = 0; m < M; ++m) {
-                            acc[m][t] = __builtin_fma((double)w[m][q].x, (double)xv.x, acc[m][t]);
-                            acc[m][t] = __builtin_fma((double)w[m][q].y, (double)xv.y, acc[m][t]);
-                            acc[m][t] = __builtin_fma((double)w[m][q].z, (double)xv.z, acc[m][t]);
-                            acc[m][t] = __builtin_fma((double)w[m][q].w, (double)xv.w, acc[m][t]);
-                        }
-                    }
-                }
-            }
-        } else {
-            for (uint32_t c = lane; c < a.cols; c += 64) {
-                float w[M];
-#pragma unroll
-                for (int m = 0; m < M; ++m) w[m] = wr[m][c];
-#pragma unroll
-                for (uint32_t t = 0; t < kMaxTokens; ++t) {
-                    if (t >= nt) break;
-                    const double xv = (double)a.x[(size_t)(t0 + t) * a.x_stride + c];
-#pragma unroll
-                    for (int m = 0; m < M; ++m)
-                        acc[m][t] = __builtin_fma((double)w[m], xv, acc[m][t]);
-                }
+                for (int m = 0; m < M; ++m) acc[m][t] = __builtin_fma((double)w[m], xv, acc[m][t]);
             }
         }
 #pragma unroll
@@ -147,6 +112,163 @@ __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
                 ys[a.y_stride + r] = act_lo_bf16(v[0], hi);
             } else {
                 a.y[at] = situ(v[0], v[M - 1], a.beta, a.has_linear, a.linear);
+            }
+        }
+    }
+}
+
+// The vector form (16-byte loads: cols and strides multiples of 4, rows
+// 16-byte aligned).  A wave takes two matrix rows (a gate / up pair, or two
+// output rows), so a lane's x values, staged in LDS kCols columns at a time
+// by the workgroup, are read and converted to double once for both; the
+// weights are non-temporal (read once a call) and eight 16-byte loads a lane
+// are in flight.  Lane l sums columns 4 (64 i + l) .. + 3, i ascending.
+// Bound: HBM.  Measured (7168 columns, one token) against a row a wave with x
+// read from the cache beside every weight: the gate/up of 6144 rows and a
+// 3584-row matrix 3.5 and 3.2 TB/s in two launches, 6.6 in one; two down
+// matrices 4.5 and 4.3 TB/s, 6.4 in one.
+// A launch runs one job or two (workgroups of job 0 first): independent
+// products fill the device together.
+enum JobOut { kOutPlain, kOutSplit, kOutSitu, kOutSum };
+
+struct VecJob {
+    JobOut out;
+    uint32_t rows, cols;
+    const float* W;
+    const float* x;
+    uint32_t x_stride;
+    // kOutSitu: the up matrix (same x).  kOutSum: y = W x + W2 x2 (each
+    // product rounded to fp32 first, then a float add).
+    const float* W2;
+    uint32_t cols2;
+    const float* x2;
+    uint32_t x2_stride;
+    float* y;
+    uint32_t y_stride;
+    uint16_t* ys;  // kOutSplit, [T][2 * y_stride]
+    float beta, linear;
+    int has_linear;
+};
+
+struct VecArgs {
+    VecJob job[2];
+    uint32_t blocks0;  // workgroups of job 0
+    uint32_t T;
+    const uint32_t* status;
+};
+
+constexpr uint32_t kCols = 1024;
+
+// acc[r][t] += w[r] . x[t] over cols columns, by the whole workgroup.
+template <int NT>
+__device__ inline void dot_rows(const float* const (&w)[2], uint32_t cols, const float* x,
+                                uint32_t x_stride, uint32_t nt, f32x4 (&s_x)[NT][kCols / 4],
+                                double (&acc)[2][NT]) {
+    const uint32_t lane = threadIdx.x & 63;
+    for (uint32_t c0 = 0; c0 < cols; c0 += kCols) {
+        const uint32_t cx = c0 + threadIdx.x * 4;
+        f32x4 xv[NT], wv[2][4];
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+            xv[t] = cx < cols && (uint32_t)t < nt
+                        ? *reinterpret_cast<const f32x4*>(x + (size_t)t * x_stride + cx)
+                        : f32x4{0.f, 0.f, 0.f, 0.f};
+        if (c0 + kCols <= cols) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int q = 0; q < 4; ++q)
+                    wv[r][q] = __builtin_nontemporal_load(
+                        reinterpret_cast<const f32x4*>(w[r] + c0 + (q * 64 + lane) * 4));
+        } else {
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const uint32_t c = c0 + (q * 64 + lane) * 4;
+                    wv[r][q] = c < cols ? *reinterpret_cast<const f32x4*>(w[r] + c)
+                                        : f32x4{0.f, 0.f, 0.f, 0.f};
+                }
+        }
+        // The barriers wait for LDS only: the weights stay in flight.
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < NT; ++t) s_x[t][threadIdx.x] = xv[t];
+        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+        for (int t = 0; t < NT; ++t)
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const f32x4 v = s_x[t][q * 64 + lane];
+#pragma unroll
+                for (int i = 0; i < 4; ++i)
+#pragma unroll
+                    for (int r = 0; r < 2; ++r)
+                        acc[r][t] =
+                            __builtin_fma((double)wv[r][q][i], (double)v[i], acc[r][t]);
+            }
+    }
+}
+
+template <int NT>
+__global__ __launch_bounds__(kThreads) void f32_gemv_vec_kernel(VecArgs a) {
+    static_assert(kThreads * 4 == kCols, "a thread stages four columns a token");
+    __shared__ f32x4 s_x[NT][kCols / 4];
+    if (*(volatile const uint32_t*)a.status) return;
+    const bool second = blockIdx.x >= a.blocks0;
+    const VecJob& j = a.job[second ? 1 : 0];
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wave = (blockIdx.x - (second ? a.blocks0 : 0)) * kWaves + (threadIdx.x >> 6);
+    // Rows past the matrix repeat its last one (not stored).
+    const bool pair = j.out == kOutSitu;
+    const uint32_t r0 = pair ? wave : 2 * wave;
+    const uint32_t ra = min(r0, j.rows - 1), rb = pair ? ra : min(r0 + 1, j.rows - 1);
+    for (uint32_t t0 = 0; t0 < a.T; t0 += NT) {
+        const uint32_t nt = min(a.T - t0, (uint32_t)NT);
+        double acc[2][NT];
+        float v[2][NT], v2[2][NT];
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) acc[r][t] = 0.0;
+        const float* const w[2] = {j.W + (size_t)ra * j.cols,
+                                   (pair ? j.W2 : j.W) + (size_t)rb * j.cols};
+        dot_rows<NT>(w, j.cols, j.x + (size_t)t0 * j.x_stride, j.x_stride, nt, s_x, acc);
+#pragma unroll
+        for (int r = 0; r < 2; ++r)
+#pragma unroll
+            for (int t = 0; t < NT; ++t) v[r][t] = (float)wave_sum(acc[r][t]);
+        if (j.out == kOutSum) {
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) acc[r][t] = 0.0;
+            const float* const w2[2] = {j.W2 + (size_t)ra * j.cols2, j.W2 + (size_t)rb * j.cols2};
+            dot_rows<NT>(w2, j.cols2, j.x2 + (size_t)t0 * j.x2_stride, j.x2_stride, nt, s_x, acc);
+#pragma unroll
+            for (int r = 0; r < 2; ++r)
+#pragma unroll
+                for (int t = 0; t < NT; ++t) v2[r][t] = (float)wave_sum(acc[r][t]);
+        }
+        if (lane != 0) continue;
+#pragma unroll
+        for (int t = 0; t < NT; ++t) {
+            if ((uint32_t)t >= nt) break;
+            float* y = j.y + (size_t)(t0 + t) * j.y_stride;
+            if (pair) {
+                if (r0 < j.rows) y[r0] = situ(v[0][t], v[1][t], j.beta, j.has_linear, j.linear);
+                continue;
+            }
+#pragma unroll
+            for (int r = 0; r < 2; ++r) {
+                if (r0 + r >= j.rows) break;
+                y[r0 + r] = j.out == kOutSum ? __fadd_rn(v[r][t], v2[r][t]) : v[r][t];
+                if (j.out == kOutSplit) {
+                    const uint16_t hi = f32_to_bf16(v[r][t]);
+                    uint16_t* ys = j.ys + (size_t)(t0 + t) * 2 * j.y_stride;
+                    ys[r0 + r] = hi;
+                    ys[j.y_stride + r0 + r] = act_lo_bf16(v[r][t], hi);
+                }
             }
         }
     }
@@ -215,26 +337,29 @@ __global__ __launch_bounds__(kThreads) void mxfp4_gemv_kernel(
 
 // RMSNorm of fp32 rows (runtime/src/ops.cpp:10-18): double sum of squares,
 // inverse = 1 / sqrt(float(sum / n) + eps) in fp32, out = x * inverse * w.
-__global__ __launch_bounds__(kThreads) void rmsnorm_f32_kernel(const float* __restrict__ x,
+constexpr int kNormWaves = 16, kNormThreads = 64 * kNormWaves;
+
+__global__ __launch_bounds__(kNormThreads) void rmsnorm_f32_kernel(const float* __restrict__ x,
                                                                const float* __restrict__ w,
                                                                uint32_t n, uint32_t n_div,
                                                                float eps,
                                                                float* __restrict__ out,
                                                                const uint32_t* status) {
-    __shared__ double part[kWaves];
+    __shared__ double part[kNormWaves];
     if (*(volatile const uint32_t*)status) return;
     const float* xr = x + (size_t)blockIdx.x * n;
     double sq = 0.0;
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads) sq = __builtin_fma((double)xr[i], (double)xr[i], sq);
+    for (uint32_t i = threadIdx.x; i < n; i += kNormThreads)
+        sq = __builtin_fma((double)xr[i], (double)xr[i], sq);
     sq = wave_sum(sq);
     if ((threadIdx.x & 63) == 0) part[threadIdx.x >> 6] = sq;
     __syncthreads();
     double tot = 0.0;
 #pragma unroll
-    for (int i = 0; i < kWaves; ++i) tot += part[i];
+    for (int i = 0; i < kNormWaves; ++i) tot += part[i];
     const float inv = __fdiv_rn(1.0f, __fsqrt_rn(__fadd_rn((float)(tot / (double)n_div), eps)));
     float* orow = out + (size_t)blockIdx.x * n;
-    for (uint32_t i = threadIdx.x; i < n; i += kThreads)
+    for (uint32_t i = threadIdx.x; i < n; i += kNormThreads)
         orow[i] = __fmul_rn(__fmul_rn(xr[i], inv), w[i]);
 }
 
@@ -245,17 +370,88 @@ int launched(k3x_hip_ctx* ctx, unsigned n) {
 
 bool aligned16(const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; }
 
+bool vec_ok(const float* W, const float* x, uint32_t cols, uint32_t x_stride) {
+    return cols % 4 == 0 && x_stride % 4 == 0 && aligned16(W) && aligned16(x);
+}
+
+int launch_vec(k3x_hip_ctx* ctx, const VecJob& a, const VecJob* b, uint32_t T) {
+    VecArgs args{};
+    args.T = T;
+    args.status = ctx->status;
+    auto blocks = [](const VecJob& j) {
+        const uint32_t waves = j.out == kOutSitu ? j.rows : (j.rows + 1) / 2;
+        return (waves + kWaves - 1) / kWaves;
+    };
+    args.job[0] = a;
+    args.blocks0 = blocks(a);
+    uint32_t total = args.blocks0;
+    if (b) {
+        args.job[1] = *b;
+        total += blocks(*b);
+    }
+    if (T == 1)
+        hipLaunchKernelGGL(f32_gemv_vec_kernel<1>, dim3(total), dim3(kThreads), 0, ctx->stream, args);
+    else if (T == 2)
+        hipLaunchKernelGGL(f32_gemv_vec_kernel<2>, dim3(total), dim3(kThreads), 0, ctx->stream, args);
+    else if (T <= 4)
+        hipLaunchKernelGGL(f32_gemv_vec_kernel<4>, dim3(total), dim3(kThreads), 0, ctx->stream, args);
+    else  // passes of eight tokens
+        hipLaunchKernelGGL(f32_gemv_vec_kernel<8>, dim3(total), dim3(kThreads), 0, ctx->stream, args);
+    return launched(ctx, 1);
+}
+
 template <int OUT>
 int launch_gemv(k3x_hip_ctx* ctx, GemvArgs a, hipStream_t stream) {
-    const bool vec = a.cols % 4 == 0 && aligned16(a.W) && aligned16(a.x) && a.x_stride % 4 == 0 &&
-                     (OUT != 3 || aligned16(a.W2));
-    const dim3 grid((a.rows + kWaves - 1) / kWaves);
     a.status = ctx->status;
-    if (vec)
-        hipLaunchKernelGGL((f32_gemv_kernel<OUT, true>), grid, dim3(kThreads), 0, stream, a);
-    else
-        hipLaunchKernelGGL((f32_gemv_kernel<OUT, false>), grid, dim3(kThreads), 0, stream, a);
+    hipLaunchKernelGGL(f32_gemv_kernel<OUT>, dim3((a.rows + kWaves - 1) / kWaves), dim3(kThreads),
+                       0, stream, a);
     return launched(ctx, 1);
+}
+
+// y = W x.
+int matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, uint32_t cols, const float* x,
+           uint32_t T, float* y) {
+    if (vec_ok(W, x, cols, cols)) {
+        VecJob j{};
+        j.out = kOutPlain;
+        j.rows = rows;
+        j.cols = cols;
+        j.W = W;
+        j.x = x;
+        j.x_stride = cols;
+        j.y = y;
+        j.y_stride = rows;
+        return launch_vec(ctx, j, nullptr, T);
+    }
+    GemvArgs a{};
+    a.W = W;
+    a.rows = rows;
+    a.cols = cols;
+    a.x = x;
+    a.x_stride = cols;
+    a.T = T;
+    a.y = y;
+    a.y_stride = rows;
+    return launch_gemv<0>(ctx, a, ctx->stream);
+}
+
+// act = situ(gate x, up x) as a vector job.
+VecJob situ_job(const float* gate, const float* up, uint32_t rows, uint32_t cols, const float* x,
+                float* act, float beta, bool has_linear, float linear) {
+    VecJob j{};
+    j.out = kOutSitu;
+    j.rows = rows;
+    j.cols = cols;
+    j.W = gate;
+    j.W2 = up;
+    j.x = x;
+    j.x_stride = cols;
+    j.y = act;
+    j.y_stride = rows;
+    j.beta = beta;
+    j.has_linear = has_linear;
+    j.linear = linear;
+    return j;
 }
 
 bool dims_ok(uint32_t rows, uint32_t cols, uint32_t T) {
@@ -287,16 +483,7 @@ int k3x_hip_dense_f32_matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, ui
                              const float* x, uint32_t tokens, float* y) {
     if (!ctx || !W || !x || !y || !dims_ok(rows, cols, tokens)) return K3X_ERR_INVALID_EXTENT;
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
-    GemvArgs a{};
-    a.W = W;
-    a.rows = rows;
-    a.cols = cols;
-    a.x = x;
-    a.x_stride = cols;
-    a.T = tokens;
-    a.y = y;
-    a.y_stride = rows;
-    return launch_gemv<0>(ctx, a, ctx->stream);
+    return matvec(ctx, W, rows, cols, x, tokens, y);
 }
 
 int k3x_hip_mxfp4_matvec(k3x_hip_ctx* ctx, const uint8_t* packed, const uint8_t* scales,
@@ -319,31 +506,29 @@ int k3x_hip_dense_situ_mlp(k3x_hip_ctx* ctx, const float* gate, const float* up,
         return K3X_ERR_INVALID_EXTENT;
     // The betas are used as given, as situ_glu does (no checks there).
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
-    GemvArgs g{};
-    g.W = gate;
-    g.W2 = up;
-    g.rows = inter;
-    g.cols = hidden;
-    g.x = x;
-    g.x_stride = hidden;
-    g.T = tokens;
-    g.y = act;
-    g.y_stride = inter;
-    g.beta = situ_beta;
-    g.has_linear = has_situ_linear != 0;
-    g.linear = situ_linear_beta;
-    int st = launch_gemv<3>(ctx, g, ctx->stream);
-    if (st) return st;
-    GemvArgs d{};
-    d.W = down;
-    d.rows = out_rows;
-    d.cols = inter;
-    d.x = act;
-    d.x_stride = inter;
-    d.T = tokens;
-    d.y = y;
-    d.y_stride = out_rows;
-    return launch_gemv<0>(ctx, d, ctx->stream);
+    int st;
+    if (vec_ok(gate, x, hidden, hidden) && aligned16(up)) {
+        st = launch_vec(ctx,
+                        situ_job(gate, up, inter, hidden, x, act, situ_beta, has_situ_linear != 0,
+                                 situ_linear_beta),
+                        nullptr, tokens);
+    } else {
+        GemvArgs g{};
+        g.W = gate;
+        g.W2 = up;
+        g.rows = inter;
+        g.cols = hidden;
+        g.x = x;
+        g.x_stride = hidden;
+        g.T = tokens;
+        g.y = act;
+        g.y_stride = inter;
+        g.beta = situ_beta;
+        g.has_linear = has_situ_linear != 0;
+        g.linear = situ_linear_beta;
+        st = launch_gemv<3>(ctx, g, ctx->stream);
+    }
+    return st ? st : matvec(ctx, down, out_rows, inter, act, tokens, y);
 }
 
 int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
@@ -385,18 +570,40 @@ int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
     uint16_t* mixed_bf16 = (uint16_t*)take((size_t)T * L * 2);
     float* routed = (float*)take(f_hid);
     float* sact = (float*)take(f_sh);
+    // The shared MLP needs x only: its gate/up rides in the launch of the
+    // latent projection, its down projection in the last one.  (The scratch
+    // of `latent` and the others starts 256-byte aligned.)
+    const bool vec = vec_ok(w->routed_down, x, H, H) && vec_ok(w->routed_up, normed, L, L) &&
+                     vec_ok(w->shared_down, sact, S, S) && aligned16(w->shared_gate) &&
+                     aligned16(w->shared_up);
     // latent = routed_down . x (backend_cpu.cpp:317), with its split copy.
-    GemvArgs a{};
-    a.W = w->routed_down;
-    a.rows = L;
-    a.cols = H;
-    a.x = x;
-    a.x_stride = H;
-    a.T = T;
-    a.y = latent;
-    a.y_stride = L;
-    a.ys = latent_split;
-    if ((st = launch_gemv<2>(ctx, a, ctx->stream))) return st;
+    if (vec) {
+        VecJob l{};
+        l.out = kOutSplit;
+        l.rows = L;
+        l.cols = H;
+        l.W = w->routed_down;
+        l.x = x;
+        l.x_stride = H;
+        l.y = latent;
+        l.y_stride = L;
+        l.ys = latent_split;
+        const VecJob g = situ_job(w->shared_gate, w->shared_up, S, H, x, sact, p->situ_beta,
+                                  p->has_situ_linear != 0, p->situ_linear_beta);
+        if ((st = launch_vec(ctx, l, &g, T))) return st;
+    } else {
+        GemvArgs a{};
+        a.W = w->routed_down;
+        a.rows = L;
+        a.cols = H;
+        a.x = x;
+        a.x_stride = H;
+        a.T = T;
+        a.y = latent;
+        a.y_stride = L;
+        a.ys = latent_split;
+        if ((st = launch_gemv<2>(ctx, a, ctx->stream))) return st;
+    }
     // The experts on the latent, mixed in slot order in fp32
     // (backend_cpu.cpp:318-325): the bank's grouped path with fp32 input and
     // activations.
@@ -408,10 +615,27 @@ int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
                                          host_ids, host_contributions, mixed_bf16, &taps)))
         return st;
     // normalized = rms_norm(mixed, routed_norm) (backend_cpu.cpp:327-328).
-    hipLaunchKernelGGL(rmsnorm_f32_kernel, dim3(T), dim3(kThreads), 0, ctx->stream, mixed,
+    hipLaunchKernelGGL(rmsnorm_f32_kernel, dim3(T), dim3(kNormThreads), 0, ctx->stream, mixed,
                        w->routed_norm, L, Ln, p->rms_epsilon, normed, ctx->status);
     if ((st = launched(ctx, 1))) return st;
-    // routed = routed_up . normalized (backend_cpu.cpp:329-330).
+    // routed = routed_up . normalized (backend_cpu.cpp:329-330), shared =
+    // shared_down . sact, out = routed + shared (:331-335) in one launch.
+    if (vec) {
+        VecJob o{};
+        o.out = kOutSum;
+        o.rows = H;
+        o.cols = L;
+        o.W = w->routed_up;
+        o.x = normed;
+        o.x_stride = L;
+        o.W2 = w->shared_down;
+        o.cols2 = S;
+        o.x2 = sact;
+        o.x2_stride = S;
+        o.y = out;
+        o.y_stride = H;
+        return launch_vec(ctx, o, nullptr, T);
+    }
     GemvArgs r{};
     r.W = w->routed_up;
     r.rows = H;
