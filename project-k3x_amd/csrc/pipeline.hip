@@ -1370,6 +1370,8 @@ struct GemvArgs {
     // these weights to them in LDS first.
     const float* gamma;
     float eps;
+    // dense_rows_kernel: 16-row output blocks.
+    uint32_t nrb;
 };
 
 // Output element `at` of a dense projection from its fp32 sums (gate and up
@@ -1579,84 +1581,181 @@ __global__ __launch_bounds__(64 * W) void dense_gemv_kernel(GemvArgs a) {
     dense_gemv_body<S, D, OUT, W, SPLIT, LDSX, NORM>(a, blockIdx.x);
 }
 
-// The dense projections of more rows than the GEMV's: NB blocks of 16 output
-// rows (pairs, S = 2) x 16 MT tokens per 1024-thread workgroup, its 16 waves
-// over the K tiles (wave w takes tiles w, w + 16, ...), the partial
-// accumulators summed in wave order through LDS.  Each weight fragment meets
-// the MT row tiles; the activations come from the L2, which holds them for
-// every workgroup.
-// Bound: latency (a wave streams two to four tiles), then the L2's rate as
-// the tokens grow (every workgroup reads all of its tokens' rows: NB = 2
-// halves that for the single matrices).  K is split inside the workgroup
-// because 128 to 448 row blocks are all the workgroups such a matrix has, and
-// the narrow GEMM's full-K waves (28 to 96 workgroups) left most of the chip
-// idle.  OUT, split rows and epilogues as dense_gemv_body.
-constexpr int kRowsWaves = 16;
+// The dense projections of more rows than the GEMV's: a workgroup takes 64
+// output rows (pairs, S = 2; 16 a wave) x 16 MT tokens, its two groups of four
+// waves half of the K tiles each, and the halves meet through LDS.  Per K tile
+// a group's activation rows arrive in LDS by buffer loads that write LDS
+// directly (the row-quad layout of grouped_gemm.hip), in a ring of four tiles,
+// and each wave's weights in registers; step k multiplies tile k, then
+// requests tile k + 3, then waits until only the requests of steps k - 1 and k
+// are outstanding.  Split rows [hi | lo] take two steps a weight tile, which
+// stays in its registers for both.  OUT and epilogues as dense_gemv_body.
+// Bound: one CU's streaming rate over 56 to 112 workgroups at 64 tokens, the
+// products as the tokens grow.  With the activations read per wave from the
+// L2 instead (16 waves over K, one or two row blocks a workgroup) the L2's
+// rate bound it.  The official layer without its experts (five projections,
+// 366 MB, and the small kernels between them): 17 tokens 172 -> 155 us, 64
+// 258 -> 221, 127 353 -> 219.
+constexpr int kRowsStages = 4;
+typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
-template <int S, int NB, int MT, int OUT, bool SPLIT>
-__global__ __launch_bounds__(64 * kRowsWaves) void dense_rows_kernel(GemvArgs a) {
-    __shared__ f32x4 part[kRowsWaves][MT][NB * S][64];
+template <int N>
+__device__ inline void rows_wait_and_barrier() {
+    static_assert(N >= 0 && N < 64, "vmcnt field");
+    asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
+}
+
+__device__ inline void rows_load_lds16(__amdgpu_buffer_rsrc_t rsrc, u32x4* dst, uint32_t voffset,
+                                       uint32_t soffset) {
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)dst, 16, voffset, soffset, 0, 0);
+}
+
+template <int S, int MT, int OUT, bool SPLIT>
+__global__ __launch_bounds__(512, 1) void dense_rows_kernel(GemvArgs a) {
+    constexpr uint32_t kStage = MT * 256;  // 16-byte words per ring stage
+    constexpr uint32_t kRing = kRowsStages * kStage;
+    static_assert(8 * MT * S * 64 <= 2 * kRing || MT == 1, "the partial sums fit the rings");
+    __shared__ u32x4 s_a4[2 * kRing > 8 * MT * S * 64 ? 2 * kRing : 8 * MT * S * 64];
     if (*(volatile const uint32_t*)a.status) return;
-    const int lane = threadIdx.x & 63;
-    const uint32_t wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-    const uint32_t g = lane >> 4, n = lane & 15;
-    const uint32_t rb = blockIdx.x * NB, m0 = blockIdx.y * (16 * MT);
-    constexpr int H2 = SPLIT ? 2 : 1;  // activation halves
-    const u32x4* xr[MT];               // rows past the last repeat it (not stored)
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const uint32_t grp = wv / 4, wave = wv % 4, g = lane >> 4, n = lane & 15;
+    const uint32_t kt = __builtin_amdgcn_readfirstlane(a.kt);
+    const uint32_t nrb = __builtin_amdgcn_readfirstlane(a.nrb);
+    const uint32_t rb = min(blockIdx.x * 4 + wave, nrb - 1), m0 = blockIdx.y * (16 * MT);
+    const uint32_t rows = min(a.tokens - m0, (uint32_t)(16 * MT));
+    const uint32_t kb = grp * (kt / 2);  // this group's kt / 2 tiles; an odd last one below
+    constexpr uint32_t TERMS = SPLIT ? 2 : 1;
+    const uint32_t steps = kt / 2 * TERMS;
+    // This chunk's rows, and this row block's tiles.
+    const __amdgpu_buffer_rsrc_t arsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint16_t*>(a.x + (size_t)m0 * a.x_stride), (short)0, rows * a.x_stride * 2,
+        0x00020000);
+    const __amdgpu_buffer_rsrc_t wrsrc = __builtin_amdgcn_make_buffer_rsrc(
+        const_cast<uint4*>(a.tiles + (size_t)rb * kt * S * 256), (short)0, kt * S * 4096,
+        0x00020000);
+    const uint32_t lane16 = lane * 16;
+    u32x4* const ring = s_a4 + grp * kRing;
+    uint32_t aoff[MT], apos[4];
 #pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-        xr[mt] = reinterpret_cast<const u32x4*>(
-            a.x + (size_t)min(m0 + 16 * mt + n, a.tokens - 1) * a.x_stride + 32 * g);
-    const u32x4* wt = reinterpret_cast<const u32x4*>(a.tiles) + (size_t)rb * a.kt * S * 256 + lane;
-    f32x4 acc[MT][NB * S];
-#pragma unroll
-    for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-        for (int w = 0; w < NB * S; ++w) acc[mt][w] = f32x4{0.f, 0.f, 0.f, 0.f};
-    for (uint32_t k = wave; k < a.kt; k += kRowsWaves) {
-        u32x4 b[NB * S][4];
-#pragma unroll
-        for (int w = 0; w < NB * S; ++w)
-#pragma unroll
-            for (int u = 0; u < 4; ++u)
-                b[w][u] = wt[(((size_t)(w / S) * a.kt + k) * S + w % S) * 256 + u * 64];
-#pragma unroll
-        for (int h = 0; h < H2; ++h)
-#pragma unroll
-            for (int j = 0; j < 4; ++j) {
-                u32x4 xv[MT];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-                    xv[mt] = xr[mt][(size_t)k * 16 + j + (h ? a.x_lo / 8 : 0)];
-#pragma unroll
-                for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                    for (int w = 0; w < NB * S; ++w)
-                        acc[mt][w] = mfma16x16x32(as_bf16x8(xv[mt]), as_bf16x8(b[w][j]),
-                                                  acc[mt][w]);
-            }
+    for (int q = 0; q < MT; ++q) {
+        const uint32_t quad = wave * MT + q;  // rows past the last repeat it (not stored)
+        aoff[q] = (min(4 * quad + (lane & 3), rows - 1) * a.x_stride +
+                   ((lane >> 2) ^ (quad & 3)) * 8) * 2;
     }
 #pragma unroll
+    for (int j = 0; j < 4; ++j)
+        apos[j] = (n >> 2) * 64 + ((4 * g + j) ^ (n >> 2)) * 4 + (n & 3);
+    f32x4 acc[MT][S];
+#pragma unroll
     for (int mt = 0; mt < MT; ++mt)
 #pragma unroll
-        for (int w = 0; w < NB * S; ++w) part[wave][mt][w][lane] = acc[mt][w];
-    __syncthreads();
-    // Thread 16 r + c finishes row r of the chunk, column c of each block:
-    // lane 16 (r % 16 / 4) + c, element r % 4 of row tile r / 16.
-    const uint32_t r = threadIdx.x / 16, c = threadIdx.x % 16, t = m0 + r;
-    if (r >= 16 * MT || t >= a.tokens) return;
-    const uint32_t pl = 16 * (r % 16 / 4) + c, pi = r % 4, pm = r / 16;
+        for (int w = 0; w < S; ++w) acc[mt][w] = f32x4{0.f, 0.f, 0.f, 0.f};
+    constexpr int WR = SPLIT ? 2 : kRowsStages;  // weight tiles held
+    u32x4 bc[WR][S][4];
+    const uint32_t slast = steps - 1;
+#define ROWS_LOAD_A(s, buf)                                                                \
+    _Pragma("unroll") for (int q = 0; q < MT; ++q)                                         \
+        rows_load_lds16(arsrc, &ring[(buf) * kStage + (wave * MT + q) * 64], aoff[q],      \
+                        (kb + (s) / TERMS) * 256 +                                          \
+                            (SPLIT && ((s) & 1) ? a.x_lo * 2 : 0));
+#define ROWS_LOAD_B(d, s)                                                                  \
+    _Pragma("unroll") for (int w = 0; w < S; ++w) _Pragma("unroll") for (int u = 0; u < 4; ++u) \
+        bc[d][w][u] = __builtin_amdgcn_raw_buffer_load_b128(                               \
+            wrsrc, lane16, (((kb + (s) / TERMS) * S + w) * 4 + u) * 1024, 0);
+    constexpr int kW = S * 4;
+    if (steps) {
 #pragma unroll
-    for (int i = 0; i < NB; ++i) {
-        float v[S];
+        for (int d = 0; d < kRowsStages - 1; ++d) {
+            ROWS_LOAD_A(min((uint32_t)d, slast), d)
+            if (!SPLIT || d % 2 == 0) {
+                ROWS_LOAD_B(SPLIT ? d / 2 : d, min((uint32_t)d, slast))
+            }
+            asm volatile("" ::: "memory");
+        }
+        // Steps -2 and -1 may stay in flight.
+        rows_wait_and_barrier<2 * MT + (SPLIT ? 1 : 2) * kW>();
+    }
+    for (uint32_t s0 = 0; s0 < steps; s0 += kRowsStages) {
+#pragma unroll
+        for (int d = 0; d < kRowsStages; ++d) {
+            const uint32_t s = s0 + d;
+            const u32x4* sa = ring + d * kStage;
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                u32x4 av[MT];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) av[mt] = sa[mt * 256 + apos[j]];
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int w = 0; w < S; ++w)
+                        acc[mt][w] = mfma16x16x32(as_bf16x8(av[mt]),
+                                                  as_bf16x8(bc[SPLIT ? d / 2 : d][w][j]),
+                                                  acc[mt][w]);
+            }
+            if (s == slast) break;  // workgroup-uniform
+            ROWS_LOAD_A(min(s + 3, slast), (d + 3) % kRowsStages)
+            if (!SPLIT || d % 2 == 1) {
+                ROWS_LOAD_B(SPLIT ? d / 2 : (d + 3) % kRowsStages, min(s + 3, slast))
+            }
+            rows_wait_and_barrier<2 * MT + (SPLIT ? 1 : 2) * kW>();
+        }
+    }
+#undef ROWS_LOAD_A
+#undef ROWS_LOAD_B
+    asm volatile("s_waitcnt vmcnt(0) lgkmcnt(0)\n\ts_barrier" ::: "memory");
+    if (kt % 2 && grp == 0) {
+        // The last tile of an odd count, straight from memory.
+#pragma unroll
+        for (uint32_t h = 0; h < TERMS; ++h)
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                u32x4 b[S];
+#pragma unroll
+                for (int w = 0; w < S; ++w)
+                    b[w] = __builtin_amdgcn_raw_buffer_load_b128(
+                        wrsrc, lane16, (((kt - 1) * S + w) * 4 + j) * 1024, 0);
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt) {
+                    const u32x4 x = *reinterpret_cast<const u32x4*>(
+                        a.x + (size_t)(m0 + min(16 * mt + n, rows - 1)) * a.x_stride +
+                        (kt - 1) * 128 + 32 * g + 8 * j + (h ? a.x_lo : 0));
+#pragma unroll
+                    for (int w = 0; w < S; ++w)
+                        acc[mt][w] = mfma16x16x32(as_bf16x8(x), as_bf16x8(b[w]), acc[mt][w]);
+                }
+            }
+    }
+    // Group 0 finishes the first row tiles, group 1 the others: each hands
+    // the other its partial sums of them.
+    f32x4* const part = reinterpret_cast<f32x4*>(s_a4);
+    constexpr int kOwn = (MT + 1) / 2;  // group 0's row tiles
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt)
+        if ((mt < kOwn) != (grp == 0))
+#pragma unroll
+            for (int w = 0; w < S; ++w) part[((mt * S + w) * 4 + wave) * 64 + lane] = acc[mt][w];
+    __syncthreads();
+    if (blockIdx.x * 4 + wave >= nrb) return;
+#pragma unroll
+    for (int mt = 0; mt < MT; ++mt) {
+        if ((mt < kOwn) != (grp == 0)) continue;
+        f32x4 sum[S];
 #pragma unroll
         for (int w = 0; w < S; ++w) {
-            v[w] = part[0][pm][i * S + w][pl][pi];
-#pragma unroll
-            for (int q = 1; q < kRowsWaves; ++q)
-                v[w] = __fadd_rn(v[w], part[q][pm][i * S + w][pl][pi]);
+            const f32x4 o = part[((mt * S + w) * 4 + wave) * 64 + lane];
+            sum[w] = grp == 0 ? acc[mt][w] + o : o + acc[mt][w];
         }
-        store_dense<OUT, S>(a, (size_t)t * a.out_stride + (size_t)(rb + i) * 16 + c, v);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+            const uint32_t t = m0 + 16 * mt + 4 * g + i;
+            if (t >= a.tokens) continue;
+            float v[S];
+#pragma unroll
+            for (int w = 0; w < S; ++w) v[w] = sum[w][i];
+            store_dense<OUT, S>(a, (size_t)t * a.out_stride + (size_t)rb * 16 + n, v);
+        }
     }
 }
 
@@ -1741,9 +1840,11 @@ using k3x_hip::begin_stage;
 using k3x_hip::end_stage;
 
 // Tokens from which the wide grouped GEMM takes routed experts at all, and
-// dense projections.
+// dense projections (the official layer without its experts, rows kernel /
+// wide: 192 tokens 342 / 515 us, 331 492 / 527, 512 599 / 563; the whole
+// layer, where they run beside the experts, is level from 256).
 constexpr uint32_t kWideMinTokens = 128;
-constexpr uint32_t kDenseWideTokens = 128;
+constexpr uint32_t kDenseWideTokens = 256;
 
 // Lays the per-call buffers out in the context scratch; returns bytes needed
 // (base == nullptr only measures).
@@ -2851,16 +2952,18 @@ bool dense_wide_ok(WideKind kind, uint32_t N, uint32_t K, uint32_t T) {
 }
 
 template <int S, int OUT, bool SPLIT>
-int launch_dense_rows(k3x_hip_ctx* ctx, const GemvArgs& g, uint32_t N, hipStream_t stream) {
-    if (g.tokens <= 32) {
-        hipLaunchKernelGGL((dense_rows_kernel<S, 1, 2, OUT, SPLIT>), dim3(N / 16),
-                           dim3(64 * kRowsWaves), 0, stream, g);
-    } else {
-        constexpr int NB = 3 - S;  // N % 32 == 0 (checked by the callers)
-        hipLaunchKernelGGL((dense_rows_kernel<S, NB, 4, OUT, SPLIT>),
-                           dim3(N / 16 / NB, (g.tokens + 63) / 64), dim3(64 * kRowsWaves), 0,
-                           stream, g);
-    }
+int launch_dense_rows(k3x_hip_ctx* ctx, GemvArgs g, uint32_t N, hipStream_t stream) {
+    g.nrb = N / 16;
+    const uint32_t bx = (g.nrb + 3) / 4;
+    // A chunk's rows and a row block's tiles are addressed in 32 bits.
+    if ((uint64_t)g.x_stride * 64 * 2 >= (1ull << 32) || (uint64_t)g.kt * S * 4096 >= (1ull << 32))
+        return K3X_ERR_INVALID_EXTENT;
+    if (g.tokens <= 32)
+        hipLaunchKernelGGL((dense_rows_kernel<S, 2, OUT, SPLIT>), dim3(bx), dim3(512), 0, stream,
+                           g);
+    else
+        hipLaunchKernelGGL((dense_rows_kernel<S, 4, OUT, SPLIT>), dim3(bx, (g.tokens + 63) / 64),
+                           dim3(512), 0, stream, g);
     return launched(ctx, 1);
 }
 

@@ -8,7 +8,9 @@ wide GEMM's ranges.
 * The official layer's projections (bf16 latent, split activations, fp32
   routed and shared rows, the output formula): a batch against the same
   tokens run at most 16 at a time on the GEMVs.  The latent differs by one
-  bf16 ulp at most (two fp32 sums of one value, each rounded once); what that
+  bf16 ulp at most beyond what the two fp32 sums differ by (each within 2^-16
+  sum |w x| <= 2^-16 |w| |x| of the exact one; |w| <= 1.5 * 0.02 sqrt(H) for
+  the synthetic rows), which shows where a sum cancels to near zero; what that
   moves downstream is a rounding here and there, below 2^-7 in relative error
   norm as for the layer's other kernels.
 """
@@ -122,6 +124,7 @@ def test_official_rows_match_gemv(hip, T):
         rel = float((got - want).norm() / want.norm())
         assert rel <= 2.0 ** -7, (name, rel)
         if name == "latent":
-            assert ((got - want).abs() <= 2.0 ** -7 * want.abs()).all()
+            sums = 2 * 2.0 ** -16 * 1.5 * 0.02 * H ** 0.5 * hidden.double().norm(dim=1, keepdim=True)
+            assert ((got - want).abs() <= 2.0 ** -7 * want.abs() + sums).all()
     off.close()
     bank.close()
