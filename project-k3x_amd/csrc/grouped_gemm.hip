@@ -16,7 +16,11 @@
 //     XOR or padded layouts take about 1.4x as long;
 //   * each wave dequantises its weight fragments once (v_cvt_scalef32_pk_
 //     bf16_fp4 per code byte) and feeds each to the MFMAs of the chunk's
-//     eight 16-row tiles (four when the chunk has at most 64 rows);
+//     16-row tiles.  A launch's ring and activation requests hold no more row
+//     tiles than its size class (8, 6, 4 or 2; with 128 rows requested
+//     whatever the class, and no odd counts, uniform 48 rows an expert took
+//     1339 us gate/up at 7168 x 2048 instead of 1152, 64 rows 1403 instead of
+//     1328; the layer at 1024 tokens 2126 instead of 2044);
 //   * software pipeline: step k multiplies tile k, then requests activation
 //     and weight tile k + 3, then waits until only the requests of steps
 //     k - 1 and k are outstanding (the vector-memory counter retires in issue
@@ -46,9 +50,6 @@ namespace {
 constexpr int kWaves = 8;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kMTiles = kWideRows / 16;          // MFMA row tiles per chunk
-constexpr int kTileChunks = kWideRows * 16;      // 16-byte chunks per activation tile
-constexpr int kALoads = kTileChunks / kThreads;  // LDS-direct loads per wave per tile
-static_assert(kALoads * kThreads == kTileChunks, "whole activation tile per step");
 
 __device__ inline uint32_t prior_status(const uint32_t* status) { return *status; }
 __device__ inline uint32_t wave_index() {
@@ -66,12 +67,13 @@ constexpr int scale_step() {
     return Q ? 2 : 0;
 }
 
-// Vector-memory requests one wave issues at pipeline step k (activation tile,
+// Vector-memory requests one wave issues at pipeline step k (AL of the
+// activation tile,
 // q8 scale dwords, weight tile; the MXFP4 scale dwords cover four K tiles and
 // are requested at steps with k % 4 == scale_step).
-template <bool FP4, int NT, int S, int U, bool Q>
+template <bool FP4, int NT, int S, int U, bool Q, int AL>
 constexpr int step_loads(int d) {
-    return kALoads + (Q ? 1 : 0) + NT * S * U + ((FP4 && d == scale_step<Q>()) ? NT * S : 0);
+    return AL + (Q ? 1 : 0) + NT * S * U + ((FP4 && d == scale_step<Q>()) ? NT * S : 0);
 }
 
 // Waits until at most N of this wave's vector-memory requests are
@@ -86,9 +88,9 @@ __device__ inline void wait_and_barrier() {
 
 // End of pipeline step d (= k % 4): only the requests of steps k - 1 and k
 // may stay outstanding.  d is a constant once the step loop is unrolled.
-template <bool FP4, int NT, int S, int U, bool Q>
+template <bool FP4, int NT, int S, int U, bool Q, int AL>
 __device__ inline void end_step(int d) {
-#define K3X_SL(i) step_loads<FP4, NT, S, U, Q>(i)
+#define K3X_SL(i) step_loads<FP4, NT, S, U, Q, AL>(i)
     switch (d) {
         case 0: wait_and_barrier<K3X_SL(3) + K3X_SL(0)>(); break;
         case 1: wait_and_barrier<K3X_SL(0) + K3X_SL(1)>(); break;
@@ -114,10 +116,19 @@ __device__ inline void end_step(int d) {
 template <bool FP4, bool GATEUP, int NT, bool SPLIT, bool Q, int MTC = 0>
 __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
     static_assert(!Q || (FP4 && !SPLIT), "q8 rows meet MXFP4 weights, one term pair per tile");
-    // 128 KiB ring; the split gate/up's epilogue stages 128 rows of fp32
-    // values in one pass, 16 bytes of pitch padding a row more than that.
+    // The launch's row tiles (the most of a shared kind's chunks): the ring,
+    // and the activation requests of a step, hold no more rows than that.
+    constexpr int kMaxT = MTC > 0 ? MTC : kMTiles;
+    constexpr int kTileChunks = kMaxT * 256;            // 16-byte chunks per activation tile
+    constexpr int kALoads = kTileChunks / kThreads;     // LDS-direct loads per wave per tile
+    static_assert(kALoads * kThreads == kTileChunks, "whole activation tile per step");
+    // A ring of kWideStages tiles; the split gate/up's epilogue stages its
+    // rows of fp32 values in one pass, the others 16 rows at least (16 bytes
+    // of pitch padding a row).
     constexpr uint32_t kRingChunks = kWideStages * kTileChunks;
-    constexpr uint32_t kStageChunks = GATEUP && SPLIT ? kWideRows * (kWaves * NT * 4 + 1) : 0;
+    constexpr uint32_t kStageChunks = GATEUP && SPLIT ? 16 * kMaxT * (kWaves * NT * 4 + 1)
+                                      : GATEUP        ? 16 * (kWaves * NT * 2 + 1)
+                                                      : 16 * (kWaves * NT * 4 + 1);
     // Down's output row of each chunk row sits past the ring (or the split
     // epilogue's staging) in the same LDS array: as a second LDS variable it
     // made the compiler's wait counting fall back to a full drain of the
@@ -188,19 +199,19 @@ __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
         FP4 ? (uint32_t)(a.scales_per_expert * 4) : 0u, 0x00020000);
     const uint32_t lane16 = lane * 16, lane4 = lane * 4;
 
-    // Activation tile loads: wave w's load q fills the row quad 4 w + q
-    // (rows 16 w + 4 q .. + 3, 1 KiB: lane l writes row 16 w + 4 q + l % 4 at
-    // position l / 4, which holds the row's 16-byte chunk (l / 4) ^ q).  Rows
-    // past the chunk's end repeat its last row (they are never stored).
+    // Activation tile loads: wave w's load q fills the row quad kALoads w + q
+    // (four rows, 1 KiB: lane l writes row 4 quad + l % 4 at position l / 4,
+    // which holds the row's 16-byte chunk (l / 4) ^ (quad % 4)).  Rows past
+    // the chunk's end repeat its last row (they are never stored).
     const __amdgpu_buffer_rsrc_t arsrc =
         __builtin_amdgcn_make_buffer_rsrc(const_cast<uint16_t*>(a.a), (short)0, a.a_bytes, 0x00020000);
     uint32_t aoff[kALoads];
 #pragma unroll
     for (int q = 0; q < kALoads; ++q) {
-        const uint32_t r = 16 * wave + 4 * q + (lane & 3);
+        const uint32_t quad = kALoads * wave + q, r = 4 * quad + (lane & 3);
         const uint32_t rr = off + m0 + min(r, rows - 1);
         const uint32_t src = a.gather ? a.pair_token[rr] : rr;
-        aoff[q] = (src * a.a_stride + ((lane >> 2) ^ q) * 8) * 2;
+        aoff[q] = (src * a.a_stride + ((lane >> 2) ^ (quad & 3)) * 8) * 2;
     }
     // Q: scale loads also write LDS directly, one dword per lane: waves w
     // and w + 4 both fill quarter w % 4 of a stage (rows 32 (w % 4) ..
@@ -245,9 +256,8 @@ __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
     // unrolled loops, so they live in registers.
 #define WIDE_LOAD_A(k, buf)                                                                  \
     _Pragma("unroll") for (int q = 0; q < kALoads; ++q)                                      \
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(                                            \
-            arsrc, (lds_ptr_t)&s_a4[(buf) * kTileChunks + (16 * wave + 4 * q) * 16], 16,      \
-            aoff[q], (kSplitIn ? ((k) & 1) * kt + ((k) >> 1) : (k)) * 256, 0, 0);
+        load_lds16(arsrc, &s_a4[(buf) * kTileChunks + (kALoads * wave + q) * 64], aoff[q],     \
+                   (kSplitIn ? ((k) & 1) * kt + ((k) >> 1) : (k)) * 256);
 #define WIDE_LOAD_B(d, k)                                                                    \
     _Pragma("unroll") for (int nt = 0; nt < NT; ++nt)                                        \
         _Pragma("unroll") for (int w = 0; w < S; ++w) {                                      \
@@ -401,7 +411,7 @@ __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
                     WIDE_LOAD_SCALES(scn, wtile(min(kb + 4, kta - 1)))
                 // Tile k + 1 (requested at step k - 2) is in LDS once only
                 // steps k - 1 and k are outstanding.
-                end_step<FP4, NT, S, U, Q>(d);
+                end_step<FP4, NT, S, U, Q, kALoads>(d);
             }
             if constexpr (FP4) {
 #pragma unroll
@@ -489,10 +499,11 @@ __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
             }
         }
     };
-    // Routed kinds: the launch's class fixes the row tiles, one step loop a
-    // kernel (with a choice of three or four row-tile counts inside one
-    // kernel, the register allocator spilled in the routed gate/up's step
-    // loop).  Shared kinds: four, six or eight row tiles, by the chunk's rows.
+    // Routed kinds: the launch's class fixes the row tiles, or one fewer where
+    // the chunk's rows allow (the classes past 64 rows keep one step
+    // loop: with a second one the register allocator spilled in it, as it did
+    // with three or four counts in any of them).  Shared kinds: four, six or eight
+    // row tiles, by the chunk's rows.
     if constexpr (MTC > 0) {
         // The grouping's class rule bounds the chunk's rows; a chunk past it
         // would lose rows, so it is an error, never a silent result.
@@ -501,7 +512,10 @@ __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
                 atomicCAS(const_cast<uint32_t*>(a.status), 0u, (uint32_t)K3X_ERR_INVALID_STATE);
             return;
         }
-        run(std::integral_constant<int, MTC>{});
+        if (MTC <= 4 && rows <= 16u * (MTC - 1))
+            run(std::integral_constant<int, MTC <= 4 ? MTC - 1 : MTC>{});
+        else
+            run(std::integral_constant<int, MTC>{});
     } else {
         static_assert(!FP4, "routed kinds launch per size class");
         if (rows > kWideRows * 3 / 4)

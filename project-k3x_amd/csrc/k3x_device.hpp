@@ -77,6 +77,15 @@ __device__ inline f32x4 mfma16x16x32(bf16x8 a, bf16x8 b, f32x4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_bf16(a, b, c, 0, 0, 0);
 }
 
+// 16 bytes a lane from a buffer resource straight to LDS at dst + 16 * lane
+// (dst wave-uniform).  A function of its own: with the cast inside a template,
+// dependent on its parameters, the host pass drops the kernel.
+__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t rsrc, u32x4* dst, uint32_t voffset,
+                                  uint32_t soffset) {
+    typedef __attribute__((address_space(3))) void* lds_ptr_t;
+    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)dst, 16, voffset, soffset, 0, 0);
+}
+
 typedef __attribute__((ext_vector_type(8))) int i32x8;
 
 // 32 E4M3 codes of one lane (two 16-byte pieces, element i in byte i) as the

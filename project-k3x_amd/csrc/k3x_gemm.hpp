@@ -126,7 +126,7 @@ struct StreamGemmArgs {
 constexpr uint32_t kStreamRows = 64;
 
 // Enqueues one launch: the records' gate/up + GLU (gateup) or down, at most
-// max_recs records of at most max_rows rows each.
+// max_recs records; max_rows: the most rows an expert can have (the tokens).
 int launch_stream_gemm(k3x_hip_ctx* ctx, bool gateup, const StreamGemmArgs& a, uint32_t max_recs,
                        uint32_t max_rows, hipStream_t stream = nullptr);
 

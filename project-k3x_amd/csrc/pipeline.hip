@@ -1597,17 +1597,11 @@ __global__ __launch_bounds__(64 * W) void dense_gemv_kernel(GemvArgs a) {
 // 366 MB, and the small kernels between them): 17 tokens 172 -> 155 us, 64
 // 258 -> 221, 127 353 -> 219.
 constexpr int kRowsStages = 4;
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
 
 template <int N>
 __device__ inline void rows_wait_and_barrier() {
     static_assert(N >= 0 && N < 64, "vmcnt field");
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-__device__ inline void rows_load_lds16(__amdgpu_buffer_rsrc_t rsrc, u32x4* dst, uint32_t voffset,
-                                       uint32_t soffset) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)dst, 16, voffset, soffset, 0, 0);
 }
 
 template <int S, int MT, int OUT, bool SPLIT>
@@ -1656,7 +1650,7 @@ __global__ __launch_bounds__(512, 1) void dense_rows_kernel(GemvArgs a) {
     const uint32_t slast = steps - 1;
 #define ROWS_LOAD_A(s, buf)                                                                \
     _Pragma("unroll") for (int q = 0; q < MT; ++q)                                         \
-        rows_load_lds16(arsrc, &ring[(buf) * kStage + (wave * MT + q) * 64], aoff[q],      \
+        load_lds16(arsrc, &ring[(buf) * kStage + (wave * MT + q) * 64], aoff[q],             \
                         (kb + (s) / TERMS) * 256 +                                          \
                             (SPLIT && ((s) & 1) ? a.x_lo * 2 : 0));
 #define ROWS_LOAD_B(d, s)                                                                  \
@@ -2573,11 +2567,9 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
         g.act_lo = split ? d.inter : 0;
         g.glu = glu;
         g.status = ctx->status;
-        // An expert takes at most one row a token.
         const uint32_t recs = small ? max_active : stream_max_records(d, T, K, srec_rows);
-        const uint32_t rec_rows = small ? T : std::min(T, srec_rows);
         mark = begin_stage(ctx, K3X_STAGE_GATE_UP);
-        st = k3x_hip::launch_stream_gemm(ctx, true, g, recs, rec_rows);
+        st = k3x_hip::launch_stream_gemm(ctx, true, g, recs, T);
         end_stage(ctx, mark);
         if (st) return st;
         g.codes = bank->dn_codes;
@@ -2596,7 +2588,7 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
         g.y_stride = d.hidden;
         g.scatter = 1;
         mark = begin_stage(ctx, K3X_STAGE_DOWN);
-        st = k3x_hip::launch_stream_gemm(ctx, false, g, recs, rec_rows);
+        st = k3x_hip::launch_stream_gemm(ctx, false, g, recs, T);
         end_stage(ctx, mark);
         if (st) return st;
         if (d.shared_inter && !side &&

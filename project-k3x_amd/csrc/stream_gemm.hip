@@ -42,20 +42,12 @@ constexpr int kWaves = 4;
 constexpr int kThreads = 64 * kWaves;
 constexpr int kStages = 4;  // ring tiles: one multiplied, three requested; a scale dword's tiles
 
-typedef __attribute__((address_space(3))) void* lds_ptr_t;
-
 // Waits until at most N of this wave's vector-memory requests are
 // outstanding and all its LDS operations are done, then meets the workgroup.
 template <int N>
 __device__ inline void wait_and_barrier() {
     static_assert(N >= 0 && N < 64, "vmcnt field");
     asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)\n\ts_barrier" ::"n"(N) : "memory");
-}
-
-// 16 bytes a lane from the resource to LDS at dst + 16 * lane.
-__device__ inline void load_lds16(__amdgpu_buffer_rsrc_t rsrc, u32x4* dst, uint32_t voffset,
-                                  uint32_t soffset) {
-    __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (lds_ptr_t)dst, 16, voffset, soffset, 0, 0);
 }
 
 template <bool GATEUP, bool SPLITIN, bool SPLITOUT, int MAXT, int NT>
@@ -339,13 +331,16 @@ void launch(const StreamGemmArgs& a, uint32_t max_recs, hipStream_t stream) {
                        0, stream, a);
 }
 
-// MAXT: the row tiles that max_rows needs, at most TMAX (records with more
-// rows are walked in chunks).
+// MAXT by the most rows an expert can have, at most TMAX (records with more
+// rows are walked in chunks).  Two row tiles up to 96 tokens: few experts have
+// more than 32 rows there, and the others gain from three workgroups a CU
+// instead of two (T=64, two / four row tiles: gate/up 6.7 / 6.4 TB/s, down 6.2
+// / 5.8; T=97 6.5 / 6.2 and 6.0 / 5.8; T=127 6.0 / 6.35 and 5.7 / 5.8).
 template <bool GATEUP, bool SPLITIN, bool SPLITOUT, int TMAX>
 void launch_tiles(const StreamGemmArgs& a, uint32_t max_recs, uint32_t max_rows,
                   hipStream_t stream) {
     if (max_rows <= 16) launch<GATEUP, SPLITIN, SPLITOUT, 1>(a, max_recs, stream);
-    else if (max_rows <= 32) launch<GATEUP, SPLITIN, SPLITOUT, 2>(a, max_recs, stream);
+    else if (max_rows <= 96) launch<GATEUP, SPLITIN, SPLITOUT, 2>(a, max_recs, stream);
     else launch<GATEUP, SPLITIN, SPLITOUT, TMAX>(a, max_recs, stream);
 }
 
