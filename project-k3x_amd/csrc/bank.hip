@@ -739,8 +739,8 @@ int k3x_hip_bank_upload_expert_device(k3x_hip_bank* bank, uint32_t expert,
         if (crc32c) expect[i] = k3x_hip::raw_of_crc(crc32c[i], len[i]);
         if (crc32c || i % 2) ext[n_ext++] = {extents[i], len[i], i, i % 2 != 0};
     }
-    int st = k3x_hip::launch_extent_check(ctx, ext, n_ext);
-    st = st ? st : retile_expert(bank, expert, extents, 0, 0, 1, expect, crc32c != nullptr);
+    if (int st = k3x_hip::launch_extent_check(ctx, ext, n_ext)) return st;  // slot untouched
+    int st = retile_expert(bank, expert, extents, 0, 0, 1, expect, crc32c != nullptr);
     if (hipStreamSynchronize(ctx->stream) != hipSuccess) st = K3X_ERR_BACKEND_UNAVAILABLE;
     if (!st)
         for (int i = 0; i < 6; ++i) {
