@@ -594,7 +594,7 @@ def storage(ctx, k3x_amd, torch, cpu: bool) -> dict:
     out = {"crc32c": {"bytes": n, "us_per_call": round(crc_s * 1e6, 1),
                       "gbps": round(n / crc_s / 1e9, 1),
                       "hbm_frac": round(n / crc_s / 1e9 / HBM_PEAK_GBS, 4),
-                      "note": "whole call: kernel, 64 Ki chunk values to the host, host fold"}}
+                      "note": "whole call: one launch, folded on the device, and its wait"}}
     del buf
 
     def dcrc(b: bytes) -> int:
