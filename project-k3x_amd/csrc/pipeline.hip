@@ -4,9 +4,11 @@
 //   router_kernel    logits = W_r xn in fp64, canonical order  (bit-exact ids)
 //   topk_kernel      sigmoid + bias, natural Top-K, renorm * routed_scale
 //   group_kernel     expert-major CSR + first-use order         (bit-exact)
-//   expert_gemm      MXFP4/bf16 weights x bf16 activations on MFMA; gate/up
+//   expert_gemm      MXFP4 weights x bf16 activations on MFMA; gate/up
 //                    variant fuses the GLU, down variant scatters per pair
-//                    (few rows per expert; many rows: grouped_gemm.hip)
+//                    (operands past 32-bit offsets; else stream_gemm.hip,
+//                    many rows grouped_gemm.hip, few tokens decode.hip)
+//   dense_*_kernel   bf16 projections: a split-K GEMV, a rows kernel
 //   combine_kernel   slot-ordered weighted sum + shared expert, bf16 cast
 #include <hip/hip_runtime.h>
 
@@ -21,6 +23,7 @@
 #include "k3x_device.hpp"
 #include "k3x_gemm.hpp"
 #include "k3x_internal.hpp"
+#include "k3x_select.hpp"
 
 using namespace k3x_dev;
 
@@ -1182,9 +1185,8 @@ __global__ __launch_bounds__(1024) void group_single_kernel(
 // Work item of one wave: NT row blocks of 16 output rows (GATEUP: NT pairs of
 // 16 gate + 16 up rows) of one expert, for all of the expert's pair rows in
 // chunks of 16*MT, over the full K.  B (weights) is read straight from the
-// tile layout into registers -- MXFP4 codes dequantised by dequant8, bf16
-// used as is -- so every weight byte is fetched once per chunk.  A
-// (activations) is read per lane from the bf16 rows the lane's MFMA row maps
+// tile layout into registers, dequantised by dequant8, so every weight byte
+// is fetched once per chunk; every offset is 64-bit.  A (activations) is read per lane from the bf16 rows the lane's MFMA row maps
 // to (gathered through pair_token for gate/up).
 //
 // Accumulator layout (16x16 MFMA): lane l, element i holds row 4(l/16)+i of
@@ -1216,6 +1218,8 @@ struct GemmArgs {
     GluParams glu;
     const uint32_t* status;
 };
+
+constexpr int kGemmDepth = 4;  // K steps in flight per wave of a one-row-tile GEMM
 
 // SPLIT: activation rows [hi | lo] (a_lo elements apart), an fp32 value in
 // two bf16 halves; each weight fragment meets both (two MFMAs, the weights
@@ -1257,46 +1261,58 @@ __global__ __launch_bounds__(256) void expert_gemm(GemmArgs a) {
 #pragma unroll
                 for (int w = 0; w < S; ++w) acc[mt][nt][w] = f32x4{0.f, 0.f, 0.f, 0.f};
 
-        for (uint32_t k = 0; k < a.kt; ++k) {
-            uint4 bt[NT][S];
-            float sc[NT][S];
-            bf16x8 af[MT][H2][4];
+        // One row tile: D K steps of loads issued together (steps past the
+        // last tile clamped, their activations zeroed), since a lone step's
+        // round trip would bound the wave.
+        constexpr int D = MT == 1 ? kGemmDepth : 1;
+        for (uint32_t k0 = 0; k0 < a.kt; k0 += D) {
+            uint4 bt[D][NT][S];
+            float sc[D][NT][S];
+            bf16x8 af[D][MT][H2][4];
 #pragma unroll
-            for (int nt = 0; nt < NT; ++nt)
-#pragma unroll
-                for (int w = 0; w < S; ++w) {
-                    bt[nt][w] = codes[(((size_t)(rb0 + nt) * a.kt + k) * S + w) * 64 + lane];
-                    const uint32_t sw =
-                        scales[(((size_t)(rb0 + nt) * a.ks + k / 4) * S + w) * 64 + lane];
-                    sc[nt][w] = e8m0_to_f32((sw >> (8 * (k & 3))) & 0xffu);
-                }
-#pragma unroll
-            for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                for (int h = 0; h < H2; ++h) {
-                    const uint4* p = reinterpret_cast<const uint4*>(
-                        arow[mt] + (h ? a.a_lo : 0u) + (size_t)k * 128);
-#pragma unroll
-                    for (int j = 0; j < 4; ++j) {
-                        const uint4 v = p[j];
-                        af[mt][h][j] = as_bf16x8(live[mt] ? v : make_uint4(0, 0, 0, 0));
-                    }
-                }
-#pragma unroll
-            for (int j = 0; j < 4; ++j)
+            for (int d = 0; d < D; ++d) {
+                const uint32_t k = min(k0 + d, a.kt - 1);
 #pragma unroll
                 for (int nt = 0; nt < NT; ++nt)
 #pragma unroll
                     for (int w = 0; w < S; ++w) {
-                        const uint4 c = bt[nt][w];
-                        const uint32_t word = j == 0 ? c.x : j == 1 ? c.y : j == 2 ? c.z : c.w;
-                        const bf16x8 b = dequant8(word, sc[nt][w]);
-#pragma unroll
-                        for (int mt = 0; mt < MT; ++mt)
-#pragma unroll
-                            for (int h = 0; h < H2; ++h)
-                                acc[mt][nt][w] = mfma16x16x32(af[mt][h][j], b, acc[mt][nt][w]);
+                        bt[d][nt][w] = codes[(((size_t)(rb0 + nt) * a.kt + k) * S + w) * 64 + lane];
+                        const uint32_t sw =
+                            scales[(((size_t)(rb0 + nt) * a.ks + k / 4) * S + w) * 64 + lane];
+                        sc[d][nt][w] = e8m0_to_f32((sw >> (8 * (k & 3))) & 0xffu);
                     }
+#pragma unroll
+                for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                    for (int h = 0; h < H2; ++h) {
+                        const uint4* p = reinterpret_cast<const uint4*>(
+                            arow[mt] + (h ? a.a_lo : 0u) + (size_t)k * 128);
+                        const bool use = live[mt] && k0 + d < a.kt;
+#pragma unroll
+                        for (int j = 0; j < 4; ++j) {
+                            const uint4 v = p[j];
+                            af[d][mt][h][j] = as_bf16x8(use ? v : make_uint4(0, 0, 0, 0));
+                        }
+                    }
+            }
+#pragma unroll
+            for (int d = 0; d < D; ++d)
+#pragma unroll
+                for (int j = 0; j < 4; ++j)
+#pragma unroll
+                    for (int nt = 0; nt < NT; ++nt)
+#pragma unroll
+                        for (int w = 0; w < S; ++w) {
+                            const uint4 c = bt[d][nt][w];
+                            const uint32_t word = j == 0 ? c.x : j == 1 ? c.y : j == 2 ? c.z : c.w;
+                            const bf16x8 b = dequant8(word, sc[d][nt][w]);
+#pragma unroll
+                            for (int mt = 0; mt < MT; ++mt)
+#pragma unroll
+                                for (int h = 0; h < H2; ++h)
+                                    acc[mt][nt][w] =
+                                        mfma16x16x32(af[d][mt][h][j], b, acc[mt][nt][w]);
+                        }
         }
 
 #pragma unroll
@@ -1830,14 +1846,17 @@ constexpr int kCombineVec = 1;  // h per thread of combine_kernel
 // ---------------------------------------------------------------------------
 
 using Scratch = k3x_hip::LayerBuffers;
+using k3x_hip::RoutedKind;
+using k3x_hip::kRoutedFew;
+using k3x_hip::kRoutedStream;
+using k3x_hip::kRoutedWide;
 using k3x_hip::begin_stage;
 using k3x_hip::end_stage;
 
-// Tokens from which the wide grouped GEMM takes routed experts at all, and
-// dense projections (the official layer without its experts, rows kernel /
-// wide: 192 tokens 342 / 515 us, 331 492 / 527, 512 599 / 563; the whole
-// layer, where they run beside the experts, is level from 256).
-constexpr uint32_t kWideMinTokens = 128;
+// Tokens from which the wide grouped GEMM takes dense projections (the
+// official layer without its experts, rows kernel / wide: 192 tokens 342 /
+// 515 us, 331 492 / 527, 512 599 / 563; the whole layer, where they run
+// beside the experts, is level from 256).
 constexpr uint32_t kDenseWideTokens = 256;
 
 // Lays the per-call buffers out in the context scratch; returns bytes needed
@@ -2243,7 +2262,7 @@ bool use_wide_gemm(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, bool spl
     constexpr uint32_t kq = 128 * k3x_hip::kWideStages;  // K extents: whole pipeline blocks
     const uint64_t rows = (uint64_t)T * K;
     // Activation and weight byte offsets are 32-bit (buffer loads).
-    return T >= kWideMinTokens && d.hidden % kq == 0 && d.inter % kq == 0 &&
+    return T >= k3x_hip::kWideMinTokens && d.hidden % kq == 0 && d.inter % kq == 0 &&
            (d.inter / 16) % wide_rb_per_block(k3x_hip::kWideRoutedGateUp) == 0 &&
            (d.hidden / 16) % wide_rb_per_block(k3x_hip::kWideRoutedDown) == 0 &&
            rows * std::max(d.hidden, d.inter * (split ? 2 : 1)) * 2 < (1ull << 32) &&
@@ -2251,36 +2270,16 @@ bool use_wide_gemm(const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, bool spl
            (uint64_t)d.inter * d.hidden * 4 < (1ull << 32);
 }
 
-// The kernels that run a call's routed experts.
-enum RoutedKind {
-    kRoutedFew,     // few tokens: the decode path's gate/up and down
-    kRoutedStream,  // the streaming GEMM (stream_gemm.hip)
-    kRoutedWide,    // many tokens: the wide GEMM (grouped_gemm.hip)
-    kRoutedNarrow,  // activation rows past 32-bit offsets: expert_gemm
-};
-
-// Tokens from which the wide GEMM's class launches beat the streaming GEMM
-// (whole layer, H=7168, 384 experts of 2048, streaming / wide: T=160 872 /
-// 1147 us, 331 1147 / 1281, 512 1484 / 1458, 768 1899 / 1773; the official
-// layer's split rows, T=331 1598 / 1867, 512 2100 / 2036).  The scaled FP4
-// path is the wide GEMM's own and keeps its range.
-constexpr uint32_t kStreamMaxTokens = 448;
-
-RoutedKind routed_kind(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank,
-                       const k3x_hip_moe_params* p) {
+k3x_hip::RoutedKind routed_kind(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank,
+                                const k3x_hip_moe_params* p) {
     const auto& d = bank->desc;
     const uint32_t T = p->tokens, K = p->top_k;
     const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
     const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
-    if (!split_in && T <= kGroupSmallTokens &&
-        k3x_hip::few_row_experts_eligible(ctx, bank, T, split))
-        return kRoutedFew;
-    if (!split_in && T >= (scaled_fp4(p) ? kWideMinTokens : kStreamMaxTokens) &&
-        use_wide_gemm(d, T, K, split))
-        return kRoutedWide;
-    const bool offsets = (uint64_t)T * d.hidden * (split_in ? 4 : 2) < (1ull << 32) &&
-                         (uint64_t)T * K * d.inter * (split ? 4 : 2) < (1ull << 32);
-    return offsets ? kRoutedStream : kRoutedNarrow;
+    return k3x_hip::select_routed(
+        {d.hidden, d.inter, T, K, split, split_in, scaled_fp4(p),
+         T <= kGroupSmallTokens && k3x_hip::few_row_experts_eligible(ctx, bank, T, split),
+         use_wide_gemm(d, T, K, split)});
 }
 
 // Arguments of the routed gate/up launch; the other three derive from them.
@@ -2627,6 +2626,8 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     mark = begin_stage(ctx, K3X_STAGE_GATE_UP);
     if (few) {
         if ((st = k3x_hip::launch_few_row_gate_up(ctx, bank, T, K, s, xn, glu, split))) return st;
+    } else if (T <= 16) {  // one row tile an expert
+        launch_gemm<true, 1, 1>(ctx, g, max_active, d.inter);
     } else {
         launch_gemm<true, 4, 1>(ctx, g, max_active, d.inter);
     }
@@ -2662,6 +2663,8 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     mark = begin_stage(ctx, K3X_STAGE_DOWN);
     if (few) {
         if ((st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split))) return st;
+    } else if (T <= 16) {
+        launch_gemm<false, 1, 2>(ctx, dn, max_active, d.hidden);
     } else {
         launch_gemm<false, 4, 2>(ctx, dn, max_active, d.hidden);
     }

@@ -353,6 +353,10 @@ int launch_stream_gemm(k3x_hip_ctx* ctx, bool gateup, const StreamGemmArgs& a, u
     if (!stream) stream = ctx->stream;
     if (!a.nrb || !a.kt || !max_recs || !max_rows || (!a.recs4 && !a.recs) || !a.n_recs)
         return K3X_ERR_INVALID_EXTENT;
+    // One expert's tiles and scales are addressed in 32 bits (stream_addressable).
+    if ((uint64_t)a.nrb * a.kt * (gateup ? 2048u : 1024u) >= (1ull << 32) ||
+        (uint64_t)a.scales_per_expert * 4 >= (1ull << 32))
+        return K3X_ERR_INVALID_EXTENT;
     // The epilogue stores 16-byte row pieces (8-byte ones for split rows).
     if (gateup ? ((uintptr_t)a.act % 16 || a.act_stride % 8 || a.act_lo % 8)
                : ((uintptr_t)a.y % 16 || a.y_stride % 4))
