@@ -28,18 +28,23 @@ int decode_forward(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_param
 // The routed experts of a general-path call on the decode path's gate/up
 // and down kernels: b.arec holds the active slots' records {expert, rows, CSR
 // offset, tokens} (the grouping writes them), act rows [P][I] or, split,
-// [P][2 I] as [hi | lo]; y receives the per-pair rows.  Whether the bank's
-// shapes and the tokens (T <= kMaxDecodeTokens) fit those kernels:
+// [P][2 I] as [hi | lo]; y receives the per-pair rows.  Few tokens (T <=
+// kMaxDecodeTokens): a slot's rows at once, tokens from the record.
+// chunked: slots of any size (T <= kChunkedMaxTokens), their rows through LDS
+// kMaxDecodeTokens at a time with the weights held in registers, tokens from
+// b.pair_token.  Whether the bank's shapes fit those kernels (T: the rows in
+// LDS at once):
+constexpr uint32_t kChunkedMaxTokens = 64;
 bool few_row_experts_eligible(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank, uint32_t T,
                               bool split);
 int launch_few_row_gate_up(k3x_hip_ctx* ctx, const k3x_hip_bank* bank, uint32_t T, uint32_t K,
                            const LayerBuffers& b, const uint16_t* xn,
-                           const k3x_dev::GluParams& glu, bool split);
+                           const k3x_dev::GluParams& glu, bool split, bool chunked = false);
 // mix (optional): the combine fused into the down launch, as on the decode
 // path (b.mix's counters, zero before and after): out = bf16(sum over slots
 // in router order of w * y (y rounded to bf16 first with round_y) +
-// shared_y), out_f32 (may be null) the same sum in fp32
-// (few_row_mix_eligible).
+// shared_y), out_f32 (may be null) the same sum in fp32.  Few tokens only
+// (few_row_mix_eligible), not chunked.
 struct FewRowMix {
     const float* weights;   // [T][K]
     const float* shared_y;  // [T][H] or null
@@ -49,7 +54,8 @@ struct FewRowMix {
 };
 bool few_row_mix_eligible(const k3x_hip_bank* bank, uint32_t T);
 int launch_few_row_down(k3x_hip_ctx* ctx, const k3x_hip_bank* bank, uint32_t T, uint32_t K,
-                        const LayerBuffers& b, bool split, const FewRowMix* mix = nullptr);
+                        const LayerBuffers& b, bool split, bool chunked = false,
+                        const FewRowMix* mix = nullptr);
 
 // out[t][h] = bf16(sum over slots in router order of w[t][s] * y[t][s][h]
 // + shared[t][h]) on the context stream (the combine of both paths).

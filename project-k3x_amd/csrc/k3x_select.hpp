@@ -9,16 +9,18 @@ namespace k3x_hip {
 
 enum RoutedKind {
     kRoutedFew,     // few tokens: the decode path's gate/up and down
+    kRoutedRows,    // few pairs: the same kernels, a slot's rows four at a time
     kRoutedStream,  // the streaming GEMM (stream_gemm.hip)
     kRoutedWide,    // many tokens: the wide GEMM (grouped_gemm.hip)
     kRoutedNarrow,  // operands past 32-bit offsets: expert_gemm
 };
 
 struct RoutedCall {
-    uint32_t hidden, inter, tokens, top_k;
+    uint32_t hidden, inter, experts, tokens, top_k;
     bool split_act, split_in;  // activation / input rows as [hi | lo] halves
     bool scaled;               // K3X_FLAG_SCALED_FP4 in effect
     bool few;                  // the decode path's kernels take these tokens
+    bool rows;                 // ... and row chunks of this shape and so many tokens
     bool wide;                 // the wide GEMM's shape rules hold
 };
 
@@ -31,6 +33,30 @@ constexpr uint32_t kWideMinTokens = 128;
 // path is the wide GEMM's own and keeps its range.
 constexpr uint32_t kStreamMaxTokens = 448;
 
+// Whether the decode kernels' row chunks beat the streaming GEMM: few pairs.
+// There a slot's workgroups split K over their eight waves and walk its rows
+// four at a time: the time grows with the pairs, and with one expert's rows
+// where few experts share them.  The streaming GEMM walks all of K in one
+// wave, a chain of tiles that a few experts' workgroups cannot hide: the
+// longer the chain (H / 128 tiles), the further both lines.  Where every token
+// takes every expert no slot has more rows than another and the line lies a
+// little further still; with one or two such experts and a long chain, 33 rows
+// make the streaming GEMM walk it twice, which the row chunks beat up to about
+// 44 rows.  Layer us over changing banks, row chunks / streaming, at (experts,
+// top_k, pairs):
+//   H=7168 I=2048  (2, 1, 5) 45 / 68, (4, 2, 10) 52 / 70, (4, 2, 22) 66 / 73,
+//                  (16, 4, 24) 88 / 93, (4, 4, 32) 69 / 72, (8, 2, 32) 80 / 74,
+//                  (1, 1, 16) 64 / 73, (1, 1, 32) 93 / 81, (1, 1, 40) 107 / 113
+//   H=3584 I=3072  (4, 2, 10) 49 / 59, (4, 2, 22) 61 / 60, (4, 2, 32) 67 / 61
+//   H=1024 I=512   (16, 2, 16) 37 / 38, (16, 4, 24) 39 / 38, (4, 2, 44) 52 / 39
+constexpr bool rows_faster(uint32_t hidden, uint32_t experts, uint32_t tokens, uint32_t top_k) {
+    const uint32_t kt = hidden / 128;
+    const bool all = experts <= top_k;
+    const uint64_t pairs = (uint64_t)tokens * top_k;
+    if (all && experts <= 2 && tokens > 32 && tokens <= kt * 4 / 5) return true;
+    return pairs <= 20 + kt / 5 + (all ? kt / 16 : 0) && pairs <= experts * (4ull + kt / 4);
+}
+
 // The streaming GEMM addresses one expert's gate/up (or down) tiles, its
 // scales and the activation rows by 32-bit byte offsets.
 constexpr bool stream_addressable(const RoutedCall& c) {
@@ -41,6 +67,8 @@ constexpr bool stream_addressable(const RoutedCall& c) {
 
 constexpr RoutedKind select_routed(const RoutedCall& c) {
     if (!c.split_in && c.few) return kRoutedFew;
+    if (!c.split_in && c.rows && rows_faster(c.hidden, c.experts, c.tokens, c.top_k))
+        return kRoutedRows;
     if (!c.split_in && c.wide && c.tokens >= (c.scaled ? kWideMinTokens : kStreamMaxTokens))
         return kRoutedWide;
     return stream_addressable(c) ? kRoutedStream : kRoutedNarrow;

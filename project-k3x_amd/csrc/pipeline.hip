@@ -1848,6 +1848,7 @@ constexpr int kCombineVec = 1;  // h per thread of combine_kernel
 using Scratch = k3x_hip::LayerBuffers;
 using k3x_hip::RoutedKind;
 using k3x_hip::kRoutedFew;
+using k3x_hip::kRoutedRows;
 using k3x_hip::kRoutedStream;
 using k3x_hip::kRoutedWide;
 using k3x_hip::begin_stage;
@@ -1990,8 +1991,9 @@ int launched(k3x_hip_ctx* ctx, unsigned n) {
 // rows (8 bits each)}, in active_asc order.
 constexpr uint32_t kGroupSmallPairs = 256;
 // Tokens up to which routes are grouped so (and with their Top-K in one
-// launch): its passes over the pairs are serial, so past the few-token calls
-// the chunked kernels are shorter (Top-K and grouping of 13 tokens, 384
+// launch) whatever their kernels, beyond only where those read its records
+// (kRoutedRows): its passes over the pairs are serial, so past the few-token
+// calls the chunked kernels are shorter (Top-K and grouping of 13 tokens, 384
 // experts, Top-16, with the router's 20 us: 72 us in one launch, 40 in two).
 constexpr uint32_t kGroupSmallTokens = 4;
 static_assert(kGroupSmallTokens * 64 <= kGroupSmallPairs, "top_k is at most 64");
@@ -2218,7 +2220,8 @@ int launch_group(k3x_hip_ctx* ctx, const uint32_t* ids, uint32_t T, uint32_t K, 
     uint32_t* chunk_fu = chunk_cnt + (size_t)nch * E;
     uint8_t* rank = reinterpret_cast<uint8_t*>(chunk_fu + (size_t)nch * E);
     const uint32_t chunk_rows = srec ? srec_rows : k3x_hip::kWideRows;
-    if (!witems && T <= kGroupSmallTokens) {
+    if (!witems && !srec && (arec || T <= kGroupSmallTokens) &&
+        (size_t)T * K <= kGroupSmallPairs) {
         hipLaunchKernelGGL(group_small_kernel, dim3(1), dim3(kGroupSmallPairs), 0, ctx->stream,
                            ids, T, K, E, ready, counts, offsets, first_use, n_active, active_asc,
                            active_fu, pair_token, pair_slot, arec, ctx->status);
@@ -2277,8 +2280,10 @@ k3x_hip::RoutedKind routed_kind(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank
     const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
     const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
     return k3x_hip::select_routed(
-        {d.hidden, d.inter, T, K, split, split_in, scaled_fp4(p),
+        {d.hidden, d.inter, d.experts, T, K, split, split_in, scaled_fp4(p),
          T <= kGroupSmallTokens && k3x_hip::few_row_experts_eligible(ctx, bank, T, split),
+         T <= k3x_hip::kChunkedMaxTokens &&
+             k3x_hip::few_row_experts_eligible(ctx, bank, k3x_hip::kMaxDecodeTokens, split),
          use_wide_gemm(d, T, K, split)});
 }
 
@@ -2453,7 +2458,7 @@ int run_wide(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
 bool shared_on_side(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_hip_moe_params* p) {
     const RoutedKind kind = routed_kind(ctx, bank, p);
     return bank->desc.shared_inter && !ctx->profiling && ctx->side_stream &&
-           (kind == kRoutedWide ||
+           (kind == kRoutedWide || kind == kRoutedRows ||
             (kind == kRoutedStream && p->tokens > (uint32_t)k3x_hip::kMaxDecodeTokens));
 }
 
@@ -2517,7 +2522,8 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     // The wide GEMM takes work items, the streaming one records: row chunks
     // (srec), or one an active expert from the small-route grouping (arec;
     // the decode path's kernels read the same records).
-    const bool small = kind != kRoutedWide && T <= kGroupSmallTokens;
+    const bool small =
+        kind == kRoutedRows || (kind != kRoutedWide && T <= kGroupSmallTokens);
     const bool chunks = kind == kRoutedStream && !small;
     const uint32_t srec_rows = stream_record_rows(d, T, K);
     uint2* const srec = reinterpret_cast<uint2*>(s.arec);
@@ -2598,7 +2604,7 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
                                        d.hidden, T, out, out_f32,
                                        (p->flags & K3X_FLAG_ROUND_EXPERT_OUT) != 0);
     }
-    const bool few = kind == kRoutedFew;
+    const bool rows = kind == kRoutedRows, few = kind == kRoutedFew || rows;
     GemmArgs g{};
     g.status = ctx->status;
     g.glu = glu;
@@ -2625,7 +2631,8 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     g.act_lo = split ? d.inter : 0;
     mark = begin_stage(ctx, K3X_STAGE_GATE_UP);
     if (few) {
-        if ((st = k3x_hip::launch_few_row_gate_up(ctx, bank, T, K, s, xn, glu, split))) return st;
+        if ((st = k3x_hip::launch_few_row_gate_up(ctx, bank, T, K, s, xn, glu, split, rows)))
+            return st;
     } else if (T <= 16) {  // one row tile an expert
         launch_gemm<true, 1, 1>(ctx, g, max_active, d.inter);
     } else {
@@ -2648,7 +2655,7 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
     dn.y_stride = d.hidden;
     // Few tokens: the combine rides in the down launch (the decode path's
     // fused mix), after the shared expert, whose output it adds.
-    if (few && k3x_hip::few_row_mix_eligible(bank, T)) {
+    if (few && !rows && k3x_hip::few_row_mix_eligible(bank, T)) {
         if (d.shared_inter && !side &&
             (st = run_shared(ctx, bank, p, s, xn, glu, ctx->stream)))
             return st;
@@ -2656,13 +2663,13 @@ int run_tail(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p,
         const k3x_hip::FewRowMix mix{weights, d.shared_inter ? s.sy : nullptr, out, out_f32,
                                      (p->flags & K3X_FLAG_ROUND_EXPERT_OUT) != 0};
         mark = begin_stage(ctx, K3X_STAGE_DOWN);
-        st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split, &mix);
+        st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split, false, &mix);
         end_stage(ctx, mark);
         return st;
     }
     mark = begin_stage(ctx, K3X_STAGE_DOWN);
     if (few) {
-        if ((st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split))) return st;
+        if ((st = k3x_hip::launch_few_row_down(ctx, bank, T, K, s, split, rows))) return st;
     } else if (T <= 16) {
         launch_gemm<false, 1, 2>(ctx, dn, max_active, d.hidden);
     } else {

@@ -21,7 +21,7 @@ def select(tmp_path_factory):
 
     def kinds(calls):
         order = ("hidden", "inter", "experts", "tokens", "top_k", "split_act", "split_in",
-                 "scaled", "few", "wide")
+                 "scaled", "few", "rows", "wide")
         text = "\n".join(" ".join(str(int(dict(BASE, **c)[f])) for f in order) for c in calls)
         return subprocess.run([exe], input=text, capture_output=True, text=True, check=True,
                               timeout=60).stdout.split()
@@ -29,7 +29,7 @@ def select(tmp_path_factory):
 
 
 BASE = dict(hidden=7168, inter=2048, experts=384, tokens=64, top_k=16, split_act=0, split_in=0,
-            scaled=0, few=0, wide=0)
+            scaled=0, few=0, rows=0, wide=0)
 
 
 @pytest.mark.parametrize("hidden,inter", [(65536, 65536), (32768, 131072), (128, 1 << 25),
@@ -50,3 +50,21 @@ def test_long_activation_rows_leave_32_bit_addressing(select):
     rows = dict(hidden=8192, inter=128, experts=8, top_k=1)
     assert select([dict(rows, tokens=(1 << 18) - 1), dict(rows, tokens=1 << 18),
                    dict(rows, tokens=1 << 17, split_in=1)]) == ["stream", "narrow", "narrow"]
+
+
+def test_few_pairs_keep_the_split_k_kernels(select):
+    """Calls of few pairs run the decode kernels' row chunks: the streaming GEMM, which walks all
+    of K in one wave, is slower there (7168 x 2048 experts, layer us row chunks / streaming: 2
+    experts, 5 tokens 45 / 68; 4 experts, Top-2, 11 tokens 66 / 73)."""
+    def kind(H, E, K, T, **more):
+        return select([dict(hidden=H, experts=E, top_k=K, tokens=T, rows=1, **more)])[0]
+    for E, K, T in ((1, 1, 5), (1, 1, 18), (1, 1, 33), (1, 1, 44), (2, 1, 30), (2, 2, 16), (2, 2, 33),
+                    (4, 2, 5), (4, 2, 13), (4, 4, 8), (16, 4, 6), (64, 4, 7), (384, 4, 5)):
+        assert kind(7168, E, K, T) == "rows", (E, K, T)
+    for E, K, T in ((1, 1, 19), (1, 1, 32), (1, 1, 45), (3, 2, 33), (8, 2, 16), (16, 8, 5), (4, 4, 9),
+                    (384, 16, 5)):
+        assert kind(7168, E, K, T) == "stream", (E, K, T)
+    assert kind(1024, 16, 4, 5) == "rows" and kind(1024, 16, 2, 11) == "stream"
+    assert kind(1024, 1, 1, 6) == "rows" and kind(1024, 1, 1, 7) == "stream"
+    assert kind(7168, 4, 2, 5, split_in=1) == "stream"
+    assert select([dict(hidden=7168, experts=4, top_k=2, tokens=5)]) == ["stream"]
