@@ -2280,7 +2280,7 @@ k3x_hip::RoutedKind routed_kind(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank
     const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
     const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
     return k3x_hip::select_routed(
-        {d.hidden, d.inter, d.experts, T, K, split, split_in, scaled_fp4(p),
+        {d.hidden, d.inter, d.experts, T, K, split, split_in, d.shared_inter != 0, scaled_fp4(p),
          T <= kGroupSmallTokens && k3x_hip::few_row_experts_eligible(ctx, bank, T, split),
          T <= k3x_hip::kChunkedMaxTokens &&
              k3x_hip::few_row_experts_eligible(ctx, bank, k3x_hip::kMaxDecodeTokens, split),

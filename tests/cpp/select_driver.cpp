@@ -1,15 +1,15 @@
 // select_driver.cpp -- prints the kernels that run a call's routed experts
 // (k3x_select.hpp), for tests/test_select.py: one call per line of stdin,
-// "hidden inter experts tokens top_k split_act split_in scaled few rows wide".
+// "hidden inter experts tokens top_k split_act split_in shared scaled few rows wide".
 #include "k3x_select.hpp"
 
 #include <cstdio>
 
 int main() {
-    unsigned h, i, e, t, k, sa, si, sc, few, rows, wide;
+    unsigned h, i, e, t, k, sa, si, sh, sc, few, rows, wide;
     const char* names[] = {"few", "rows", "stream", "wide", "narrow"};
-    while (std::scanf("%u %u %u %u %u %u %u %u %u %u %u", &h, &i, &e, &t, &k, &sa, &si, &sc, &few,
-                      &rows, &wide) == 11) {
+    while (std::scanf("%u %u %u %u %u %u %u %u %u %u %u %u", &h, &i, &e, &t, &k, &sa, &si, &sh, &sc, &few,
+                      &rows, &wide) == 12) {
         k3x_hip::RoutedCall c{};
         c.hidden = h;
         c.inter = i;
@@ -18,6 +18,7 @@ int main() {
         c.top_k = k;
         c.split_act = sa;
         c.split_in = si;
+        c.shared = sh;
         c.scaled = sc;
         c.few = few;
         c.rows = rows;

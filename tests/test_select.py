@@ -21,7 +21,7 @@ def select(tmp_path_factory):
 
     def kinds(calls):
         order = ("hidden", "inter", "experts", "tokens", "top_k", "split_act", "split_in",
-                 "scaled", "few", "rows", "wide")
+                 "shared", "scaled", "few", "rows", "wide")
         text = "\n".join(" ".join(str(int(dict(BASE, **c)[f])) for f in order) for c in calls)
         return subprocess.run([exe], input=text, capture_output=True, text=True, check=True,
                               timeout=60).stdout.split()
@@ -29,7 +29,7 @@ def select(tmp_path_factory):
 
 
 BASE = dict(hidden=7168, inter=2048, experts=384, tokens=64, top_k=16, split_act=0, split_in=0,
-            scaled=0, few=0, rows=0, wide=0)
+            shared=0, scaled=0, few=0, rows=0, wide=0)
 
 
 @pytest.mark.parametrize("hidden,inter", [(65536, 65536), (32768, 131072), (128, 1 << 25),
@@ -68,3 +68,26 @@ def test_few_pairs_keep_the_split_k_kernels(select):
     assert kind(1024, 1, 1, 6) == "rows" and kind(1024, 1, 1, 7) == "stream"
     assert kind(7168, 4, 2, 5, split_in=1) == "stream"
     assert select([dict(hidden=7168, experts=4, top_k=2, tokens=5)]) == ["stream"]
+
+
+def test_busy_experts_take_the_wide_gemm(select):
+    """From 128 tokens the choice of the wide GEMM looks at the work, not at the tokens alone:
+    few experts with many rows each fill it long before 448 tokens (16 experts of 7168 x 2048,
+    Top-16, 416 tokens: streaming 823 us, wide 598)."""
+    def kind(H, I, E, K, T, **more):
+        return select([dict(hidden=H, inter=I, experts=E, top_k=K, tokens=T, wide=1, **more)])[0]
+    for H, I, E, K, T in ((7168, 2048, 16, 16, 192), (7168, 2048, 8, 8, 300), (7168, 2048, 16, 8, 331),
+                          (7168, 2048, 64, 16, 256), (7168, 2048, 128, 16, 300),
+                          (3584, 3072, 16, 16, 192), (3584, 3072, 8, 8, 300), (4096, 1536, 16, 16, 256),
+                          (4096, 1536, 64, 16, 331), (7168, 2048, 384, 16, 448), (512, 512, 4, 1, 448)):
+        assert kind(H, I, E, K, T) == "wide", (H, I, E, K, T)
+    for H, I, E, K, T in ((7168, 2048, 16, 16, 128), (7168, 2048, 8, 8, 256), (7168, 2048, 16, 8, 256),
+                          (7168, 2048, 4, 4, 447), (7168, 2048, 8, 8, 331), (7168, 2048, 64, 16, 160), (7168, 2048, 64, 8, 300),
+                          (7168, 2048, 384, 16, 331), (3584, 3072, 896, 16, 447),
+                          (4096, 1536, 16, 8, 447), (1024, 512, 64, 16, 447)):
+        assert kind(H, I, E, K, T) == "stream", (H, I, E, K, T)
+    assert [kind(7168, 2048, 128, 16, t, shared=1) for t in (300, 352)] == ["stream", "wide"]
+    assert [kind(7168, 2048, 64, 8, t, shared=1) for t in (384, 416)] == ["stream", "wide"]
+    assert kind(7168, 2048, 384, 16, 128, scaled=1) == "wide"
+    assert kind(7168, 2048, 16, 16, 416, split_in=1) == "stream"
+    assert select([dict(tokens=4096)]) == ["stream"]
