@@ -129,7 +129,7 @@ __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
 // matrices 4.5 and 4.3 TB/s, 6.4 in one.
 // A launch runs one job or two (workgroups of job 0 first): independent
 // products fill the device together.
-enum JobOut { kOutPlain, kOutSplit, kOutSitu, kOutSum };
+enum JobOut { kOutPlain, kOutSplit, kOutSitu, kOutSum, kOutAdd };
 
 struct VecJob {
     JobOut out;
@@ -138,7 +138,8 @@ struct VecJob {
     const float* x;
     uint32_t x_stride;
     // kOutSitu: the up matrix (same x).  kOutSum: y = W x + W2 x2 (each
-    // product rounded to fp32 first, then a float add).
+    // product rounded to fp32 first, then a float add).  kOutAdd: y = x2 + W x,
+    // x2 rows of y's shape.
     const float* W2;
     uint32_t cols2;
     const float* x2;
@@ -262,7 +263,11 @@ __global__ __launch_bounds__(kThreads) void f32_gemv_vec_kernel(VecArgs a) {
 #pragma unroll
             for (int r = 0; r < 2; ++r) {
                 if (r0 + r >= j.rows) break;
-                y[r0 + r] = j.out == kOutSum ? __fadd_rn(v[r][t], v2[r][t]) : v[r][t];
+                float sum = v[r][t];
+                if (j.out == kOutSum) sum = __fadd_rn(sum, v2[r][t]);
+                if (j.out == kOutAdd)
+                    sum = __fadd_rn(j.x2[(size_t)(t0 + t) * j.x2_stride + r0 + r], sum);
+                y[r0 + r] = sum;
                 if (j.out == kOutSplit) {
                     const uint16_t hi = f32_to_bf16(v[r][t]);
                     uint16_t* ys = j.ys + (size_t)(t0 + t) * 2 * j.y_stride;
@@ -408,21 +413,21 @@ int launch_gemv(k3x_hip_ctx* ctx, GemvArgs a, hipStream_t stream) {
     return launched(ctx, 1);
 }
 
-// y = W x.
-int matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, uint32_t cols, const float* x,
-           uint32_t T, float* y) {
-    if (vec_ok(W, x, cols, cols)) {
-        VecJob j{};
-        j.out = kOutPlain;
-        j.rows = rows;
-        j.cols = cols;
-        j.W = W;
-        j.x = x;
-        j.x_stride = cols;
-        j.y = y;
-        j.y_stride = rows;
-        return launch_vec(ctx, j, nullptr, T);
-    }
+VecJob plain_job(const float* W, uint32_t rows, uint32_t cols, const float* x, float* y) {
+    VecJob j{};
+    j.out = kOutPlain;
+    j.rows = rows;
+    j.cols = cols;
+    j.W = W;
+    j.x = x;
+    j.x_stride = cols;
+    j.y = y;
+    j.y_stride = rows;
+    return j;
+}
+
+GemvArgs plain_args(const float* W, uint32_t rows, uint32_t cols, const float* x, uint32_t T,
+                    float* y) {
     GemvArgs a{};
     a.W = W;
     a.rows = rows;
@@ -432,26 +437,46 @@ int matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, uint32_t cols, const
     a.T = T;
     a.y = y;
     a.y_stride = rows;
-    return launch_gemv<0>(ctx, a, ctx->stream);
+    return a;
+}
+
+// y = W x.
+int matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, uint32_t cols, const float* x,
+           uint32_t T, float* y) {
+    if (vec_ok(W, x, cols, cols))
+        return launch_vec(ctx, plain_job(W, rows, cols, x, y), nullptr, T);
+    return launch_gemv<0>(ctx, plain_args(W, rows, cols, x, T, y), ctx->stream);
 }
 
 // act = situ(gate x, up x) as a vector job.
 VecJob situ_job(const float* gate, const float* up, uint32_t rows, uint32_t cols, const float* x,
                 float* act, float beta, bool has_linear, float linear) {
-    VecJob j{};
+    VecJob j = plain_job(gate, rows, cols, x, act);
     j.out = kOutSitu;
-    j.rows = rows;
-    j.cols = cols;
-    j.W = gate;
     j.W2 = up;
-    j.x = x;
-    j.x_stride = cols;
-    j.y = act;
-    j.y_stride = rows;
     j.beta = beta;
     j.has_linear = has_linear;
     j.linear = linear;
     return j;
+}
+
+bool situ_vec_ok(const float* gate, const float* up, const float* x, uint32_t cols) {
+    return vec_ok(gate, x, cols, cols) && aligned16(up);
+}
+
+// act = situ(gate x, up x).
+int situ_product(k3x_hip_ctx* ctx, const float* gate, const float* up, uint32_t rows,
+                 uint32_t cols, const float* x, uint32_t T, float* act, float beta, bool has_linear,
+                 float linear) {
+    if (situ_vec_ok(gate, up, x, cols))
+        return launch_vec(ctx, situ_job(gate, up, rows, cols, x, act, beta, has_linear, linear),
+                          nullptr, T);
+    GemvArgs g = plain_args(gate, rows, cols, x, T, act);
+    g.W2 = up;
+    g.beta = beta;
+    g.has_linear = has_linear;
+    g.linear = linear;
+    return launch_gemv<3>(ctx, g, ctx->stream);
 }
 
 bool dims_ok(uint32_t rows, uint32_t cols, uint32_t T) {
@@ -506,28 +531,8 @@ int k3x_hip_dense_situ_mlp(k3x_hip_ctx* ctx, const float* gate, const float* up,
         return K3X_ERR_INVALID_EXTENT;
     // The betas are used as given, as situ_glu does (no checks there).
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
-    int st;
-    if (vec_ok(gate, x, hidden, hidden) && aligned16(up)) {
-        st = launch_vec(ctx,
-                        situ_job(gate, up, inter, hidden, x, act, situ_beta, has_situ_linear != 0,
-                                 situ_linear_beta),
-                        nullptr, tokens);
-    } else {
-        GemvArgs g{};
-        g.W = gate;
-        g.W2 = up;
-        g.rows = inter;
-        g.cols = hidden;
-        g.x = x;
-        g.x_stride = hidden;
-        g.T = tokens;
-        g.y = act;
-        g.y_stride = inter;
-        g.beta = situ_beta;
-        g.has_linear = has_situ_linear != 0;
-        g.linear = situ_linear_beta;
-        st = launch_gemv<3>(ctx, g, ctx->stream);
-    }
+    const int st = situ_product(ctx, gate, up, inter, hidden, x, tokens, act, situ_beta,
+                                has_situ_linear != 0, situ_linear_beta);
     return st ? st : matvec(ctx, down, out_rows, inter, act, tokens, y);
 }
 
@@ -571,39 +576,30 @@ int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
     float* routed = (float*)take(f_hid);
     float* sact = (float*)take(f_sh);
     // The shared MLP needs x only: its gate/up rides in the launch of the
-    // latent projection, its down projection in the last one.  (The scratch
-    // of `latent` and the others starts 256-byte aligned.)
-    const bool vec = vec_ok(w->routed_down, x, H, H) && vec_ok(w->routed_up, normed, L, L) &&
-                     vec_ok(w->shared_down, sact, S, S) && aligned16(w->shared_gate) &&
-                     aligned16(w->shared_up);
+    // latent projection, its down projection in the last one, where both
+    // products of a launch take 16-byte loads; each product that does not is
+    // a launch of its own, the others keep theirs.  (The scratch of `latent`
+    // and the others starts 256-byte aligned.)
+    const bool has_linear = p->has_situ_linear != 0;
+    bool shared_done = false;
     // latent = routed_down . x (backend_cpu.cpp:317), with its split copy.
-    if (vec) {
-        VecJob l{};
+    if (vec_ok(w->routed_down, x, H, H)) {
+        VecJob l = plain_job(w->routed_down, L, H, x, latent);
         l.out = kOutSplit;
-        l.rows = L;
-        l.cols = H;
-        l.W = w->routed_down;
-        l.x = x;
-        l.x_stride = H;
-        l.y = latent;
-        l.y_stride = L;
         l.ys = latent_split;
         const VecJob g = situ_job(w->shared_gate, w->shared_up, S, H, x, sact, p->situ_beta,
-                                  p->has_situ_linear != 0, p->situ_linear_beta);
-        if ((st = launch_vec(ctx, l, &g, T))) return st;
+                                  has_linear, p->situ_linear_beta);
+        shared_done = situ_vec_ok(w->shared_gate, w->shared_up, x, H);
+        if ((st = launch_vec(ctx, l, shared_done ? &g : nullptr, T))) return st;
     } else {
-        GemvArgs a{};
-        a.W = w->routed_down;
-        a.rows = L;
-        a.cols = H;
-        a.x = x;
-        a.x_stride = H;
-        a.T = T;
-        a.y = latent;
-        a.y_stride = L;
+        GemvArgs a = plain_args(w->routed_down, L, H, x, T, latent);
         a.ys = latent_split;
         if ((st = launch_gemv<2>(ctx, a, ctx->stream))) return st;
     }
+    if (!shared_done &&
+        (st = situ_product(ctx, w->shared_gate, w->shared_up, S, H, x, T, sact, p->situ_beta,
+                           has_linear, p->situ_linear_beta)))
+        return st;
     // The experts on the latent, mixed in slot order in fp32
     // (backend_cpu.cpp:318-325): the bank's grouped path with fp32 input and
     // activations.
@@ -620,57 +616,25 @@ int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
     if ((st = launched(ctx, 1))) return st;
     // routed = routed_up . normalized (backend_cpu.cpp:329-330), shared =
     // shared_down . sact, out = routed + shared (:331-335) in one launch.
-    if (vec) {
-        VecJob o{};
+    const bool down_vec = vec_ok(w->shared_down, sact, S, S);
+    if (down_vec && vec_ok(w->routed_up, normed, L, L)) {
+        VecJob o = plain_job(w->routed_up, H, L, normed, out);
         o.out = kOutSum;
-        o.rows = H;
-        o.cols = L;
-        o.W = w->routed_up;
-        o.x = normed;
-        o.x_stride = L;
         o.W2 = w->shared_down;
         o.cols2 = S;
         o.x2 = sact;
         o.x2_stride = S;
-        o.y = out;
-        o.y_stride = H;
         return launch_vec(ctx, o, nullptr, T);
     }
-    GemvArgs r{};
-    r.W = w->routed_up;
-    r.rows = H;
-    r.cols = L;
-    r.x = normed;
-    r.x_stride = L;
-    r.T = T;
-    r.y = routed;
-    r.y_stride = H;
-    if ((st = launch_gemv<0>(ctx, r, ctx->stream))) return st;
-    // shared = dense_situ_mlp(x) (backend_cpu.cpp:331-332); out = routed +
-    // shared (:333-335) in the down projection's epilogue.
-    GemvArgs g{};
-    g.W = w->shared_gate;
-    g.W2 = w->shared_up;
-    g.rows = S;
-    g.cols = H;
-    g.x = x;
-    g.x_stride = H;
-    g.T = T;
-    g.y = sact;
-    g.y_stride = S;
-    g.beta = p->situ_beta;
-    g.has_linear = p->has_situ_linear != 0;
-    g.linear = p->situ_linear_beta;
-    if ((st = launch_gemv<3>(ctx, g, ctx->stream))) return st;
-    GemvArgs d{};
-    d.W = w->shared_down;
-    d.rows = H;
-    d.cols = S;
-    d.x = sact;
-    d.x_stride = S;
-    d.T = T;
-    d.y = out;
-    d.y_stride = H;
+    if ((st = matvec(ctx, w->routed_up, H, L, normed, T, routed))) return st;
+    if (down_vec) {
+        VecJob o = plain_job(w->shared_down, H, S, sact, out);
+        o.out = kOutAdd;
+        o.x2 = routed;
+        o.x2_stride = H;
+        return launch_vec(ctx, o, nullptr, T);
+    }
+    GemvArgs d = plain_args(w->shared_down, H, S, sact, T, out);
     d.add = routed;
     return launch_gemv<1>(ctx, d, ctx->stream);
 }
