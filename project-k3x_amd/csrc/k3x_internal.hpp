@@ -276,6 +276,8 @@ int dense_gate_up(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t I, uint32_t H, 
 // is then unused) and write the official layer's output (dense_down_output);
 // on the wide GEMM y_bf16 must be null.
 bool dense_direct(uint32_t N, uint32_t K, uint32_t T);
+// Whether they take 16-byte aligned rows (the GEMV reads any).
+bool dense_rows_to_lds(uint32_t T);
 int dense_down(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t K, const uint16_t* a,
                uint32_t T, float* y, hipStream_t stream, uint16_t* y_bf16 = nullptr,
                bool split = false);

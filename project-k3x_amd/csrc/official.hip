@@ -531,9 +531,12 @@ struct FfnBuffers {
     float* routed;        // [T][H]
     uint16_t* sact;       // [T][2 Is] split [hi | lo] rows
     float* shared;        // [T][H]
+    uint16_t* hidden;     // [T][H] aligned copy, or null
 };
 
-size_t carve(uint8_t* base, const k3x_hip_official* o, uint32_t T, uint32_t K, FfnBuffers* b) {
+// copy: room for an aligned copy of the hidden rows.
+size_t carve(uint8_t* base, const k3x_hip_official* o, uint32_t T, uint32_t K, bool copy,
+             FfnBuffers* b) {
     size_t at = 0;
     auto take = [&](size_t bytes) {
         uint8_t* p = base ? base + at : nullptr;
@@ -550,6 +553,7 @@ size_t carve(uint8_t* base, const k3x_hip_official* o, uint32_t T, uint32_t K, F
     b->routed = (float*)take((size_t)T * o->H * 4);
     b->sact = (uint16_t*)take((size_t)T * std::max(o->I_s, 1u) * 4);
     b->shared = (float*)take((size_t)T * o->H * 4);
+    b->hidden = copy ? (uint16_t*)take((size_t)T * o->H * 2) : nullptr;
     return at;
 }
 
@@ -785,9 +789,12 @@ int k3x_hip_official_ffn(k3x_hip_ctx* ctx, k3x_hip_official* o, const k3x_hip_mo
             if (!r) return K3X_ERR_INVALID_STATE;
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
     FfnBuffers b;
-    int st = ensure(o, carve(nullptr, o, T, K, &b));
+    // The projections of more rows than the GEMV's load the hidden rows
+    // straight into LDS, 16 bytes a lane: rows off that alignment go through a copy.
+    const bool copy = reinterpret_cast<uintptr_t>(hidden) % 16 && k3x_hip::dense_rows_to_lds(T);
+    int st = ensure(o, carve(nullptr, o, T, K, copy, &b));
     if (st) return st;
-    carve(static_cast<uint8_t*>(o->scratch), o, T, K, &b);
+    carve(static_cast<uint8_t*>(o->scratch), o, T, K, copy, &b);
     // Experts on the latent: the bank's grouped path with fp32 activations
     // into the down projection, each expert output rounded to bf16 before the
     // slot-ordered mix, the mix rounded (official_moe.cpp:82-103, :313-326).
@@ -798,6 +805,10 @@ int k3x_hip_official_ffn(k3x_hip_ctx* ctx, k3x_hip_official* o, const k3x_hip_mo
     k3x_hip::LayerBuffers rs;
     // Its scratch is carved (and grown) before any launch of this call.
     if ((st = k3x_hip::routed_begin(ctx, o->bank, &ep, &rs))) return st;
+    if (copy) {
+        if ((st = copy_d2d(ctx, b.hidden, hidden, (size_t)T * o->H * 2))) return st;
+        hidden = b.hidden;
+    }
     const GluParams glu{(int)p->glu, p->situ_beta, (int)p->has_situ_linear, p->situ_linear_beta};
     // Shared FFN on hidden (official_moe.cpp:105-117, :307): on the side
     // stream beside the route and the experts (few rows: the routed kernels

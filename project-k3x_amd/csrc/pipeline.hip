@@ -1899,9 +1899,10 @@ bool scaled_fp4(const k3x_hip_moe_params* p) {
 }
 
 // split: the routed activation rows hold [hi | lo] halves (K3X_FLAG_SPLIT_ACT);
-// q8: room for the q8 rows of the scaled FP4 wide GEMM.
+// split_in: xn holds [hi | lo] rows (K3X_FLAG_SPLIT_INPUT); q8: room for the q8
+// rows of the scaled FP4 wide GEMM.
 size_t carve(uint8_t* base, const k3x_hip_layer_desc& d, uint32_t T, uint32_t K, bool split,
-             bool q8, Scratch* s) {
+             bool split_in, bool q8, Scratch* s) {
     size_t at = 0;
     auto take = [&](size_t bytes) {
         uint8_t* p = base ? base + at : nullptr;
@@ -1909,7 +1910,7 @@ size_t carve(uint8_t* base, const k3x_hip_layer_desc& d, uint32_t T, uint32_t K,
         return p;
     };
     const size_t P = (size_t)T * K;
-    s->xn = (uint16_t*)take((size_t)T * d.hidden * 2);
+    s->xn = (uint16_t*)take((size_t)T * d.hidden * (split_in ? 4 : 2));
     s->logits = (float*)take((size_t)T * d.experts * 4);
     s->ids = (uint32_t*)take(P * 4);
     s->weights = (float*)take(P * 4);
@@ -2319,6 +2320,15 @@ k3x_hip::WideGemmArgs wide_gate_up_args(k3x_hip_ctx* ctx, const k3x_hip_bank* ba
     g.act_stride = split ? 2 * d.inter : d.inter;
     g.act_lo = split ? d.inter : 0;
     return g;
+}
+
+// Whether a call's kernels bring its input rows to LDS by buffer loads of 16
+// bytes a lane, which take aligned rows (the streaming and wide GEMMs, and the
+// shared expert's rows and wide kernels); the others read them with plain loads.
+bool rows_to_lds(const k3x_hip_ctx* ctx, const k3x_hip_bank* bank, const k3x_hip_moe_params* p) {
+    const RoutedKind kind = routed_kind(ctx, bank, p);
+    return kind == kRoutedStream || kind == kRoutedWide ||
+           (bank->desc.shared_inter && k3x_hip::dense_rows_to_lds(p->tokens));
 }
 
 // The shared expert: gate/up + GLU -> sact, down -> sy, on `stream` (stage
@@ -2824,11 +2834,13 @@ int launch_topk_group_impl(k3x_hip_ctx* ctx, const float* logits, const float* b
 int prepare(k3x_hip_ctx* ctx, k3x_hip_bank* bank, const k3x_hip_moe_params* p, Scratch* s) {
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
     const bool split = (p->flags & K3X_FLAG_SPLIT_ACT) != 0;
+    const bool split_in = (p->flags & K3X_FLAG_SPLIT_INPUT) != 0;
     const bool q8 = scaled_fp4(p);
-    const size_t need = carve(nullptr, bank->desc, p->tokens, p->top_k, split, q8, s);
+    const size_t need = carve(nullptr, bank->desc, p->tokens, p->top_k, split, split_in, q8, s);
     int st = k3x_hip::ensure_scratch(ctx, need);
     if (st) return st;
-    carve(static_cast<uint8_t*>(ctx->scratch), bank->desc, p->tokens, p->top_k, split, q8, s);
+    carve(static_cast<uint8_t*>(ctx->scratch), bank->desc, p->tokens, p->top_k, split, split_in, q8,
+          s);
     s->mix = ctx->mix_counts;
     return K3X_OK;
 }
@@ -3003,6 +3015,8 @@ int dense_norm_output(k3x_hip_ctx* ctx, const uint4* tiles, uint32_t N, uint32_t
                        dim3(64 * kGemvWaves), (size_t)T * K * 2 + (size_t)K * 4, ctx->stream, g);
     return launched(ctx, 1);
 }
+
+bool dense_rows_to_lds(uint32_t T) { return T > kGemvMaxTokens; }
 
 bool dense_direct(uint32_t N, uint32_t K, uint32_t T) {
     return !dense_wide_ok(kWideSharedDown, N, K, T);
@@ -3259,11 +3273,11 @@ int k3x_hip_moe_forward_noalloc(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
     // counters (zero from load time, left zero by every call); the carve
     // stays below them.
     constexpr size_t kCarveMax = K3X_HIP_NOALLOC_SCRATCH_BYTES - k3x_hip::kDecodeMixBytes;
-    if (carve(nullptr, bank->desc, p->tokens, p->top_k, split, q8, &s) > kCarveMax)
+    if (carve(nullptr, bank->desc, p->tokens, p->top_k, split, false, q8, &s) > kCarveMax)
         return K3X_ERR_INVALID_EXTENT;
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
     carve(static_cast<uint8_t*>(ctx->noalloc_scratch), bank->desc, p->tokens, p->top_k, split,
-          q8, &s);
+          false, q8, &s);
     s.mix = reinterpret_cast<uint32_t*>(static_cast<uint8_t*>(ctx->noalloc_scratch) + kCarveMax);
     // Stage timing takes events from a pool that may have to create them:
     // not on this path.
@@ -3300,6 +3314,12 @@ int k3x_hip_moe_forward_routed(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
             if (!std::isfinite(host_weights[i])) return K3X_ERR_INVALID_STATE;
     Scratch s;
     if ((st = prepare(ctx, bank, p, &s))) return st;
+    if (reinterpret_cast<uintptr_t>(xn) % 16 && rows_to_lds(ctx, bank, p)) {
+        const size_t row = (size_t)bank->desc.hidden * (p->flags & K3X_FLAG_SPLIT_INPUT ? 4 : 2);
+        if (hipMemcpyAsync(s.xn, xn, T * row, hipMemcpyDeviceToDevice, ctx->stream) != hipSuccess)
+            return K3X_ERR_BACKEND_UNAVAILABLE;
+        xn = s.xn;
+    }
     return k3x_hip::routed_finish(ctx, bank, p, s, xn, ids, weights, out, taps);
 }
 
