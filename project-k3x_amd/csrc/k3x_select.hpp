@@ -97,6 +97,12 @@ constexpr bool stream_addressable(const RoutedCall& c) {
            T * c.hidden * (c.split_in ? 4 : 2) < lim && T * K * c.inter * (c.split_act ? 4 : 2) < lim;
 }
 
+// The rows kernel of the dense projections addresses a chunk of 64 rows (stride
+// in elements) and a 16-row block's tiles by 32-bit byte offsets.
+constexpr bool dense_rows_addressable(uint64_t stride, uint64_t block_bytes) {
+    return stride * 64 * 2 < (1ull << 32) && block_bytes < (1ull << 32);
+}
+
 constexpr RoutedKind select_routed(const RoutedCall& c) {
     if (!c.split_in && c.few) return kRoutedFew;
     if (!c.split_in && c.rows && rows_faster(c.hidden, c.experts, c.tokens, c.top_k))

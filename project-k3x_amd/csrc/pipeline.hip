@@ -2965,13 +2965,34 @@ bool dense_wide_ok(WideKind kind, uint32_t N, uint32_t K, uint32_t T) {
            (uint64_t)T * std::max(N, K) * 4 < (1ull << 32) && (uint64_t)N * K * 4 < (1ull << 32);
 }
 
+// The GEMV 16 tokens at a time, for rows past the rows kernel's 32-bit offsets.
+template <int S, int OUT, bool SPLIT>
+int launch_dense_passes(k3x_hip_ctx* ctx, const GemvArgs& g, uint32_t N, hipStream_t stream) {
+    constexpr size_t kOutBytes = OUT == 0 ? 4 : 2;
+    for (uint32_t t0 = 0; t0 < g.tokens; t0 += kGemvMaxTokens) {
+        const size_t at = (size_t)t0 * g.out_stride;
+        GemvArgs p = g;
+        p.tokens = std::min(g.tokens - t0, kGemvMaxTokens);
+        p.x = g.x + (size_t)t0 * g.x_stride;
+        p.out = static_cast<uint8_t*>(g.out) + at * kOutBytes;
+        if (OUT == 3) {
+            p.prefix = g.prefix + at;
+            p.shared = g.shared ? g.shared + at : nullptr;
+            p.routed = g.routed + at;
+        }
+        hipLaunchKernelGGL((dense_gemv_kernel<S, 1, OUT, kGemvWaves / 2, SPLIT>), dim3(N / 16),
+                           dim3(32 * kGemvWaves), 0, stream, p);
+        if (const int st = launched(ctx, 1)) return st;
+    }
+    return K3X_OK;
+}
+
 template <int S, int OUT, bool SPLIT>
 int launch_dense_rows(k3x_hip_ctx* ctx, GemvArgs g, uint32_t N, hipStream_t stream) {
     g.nrb = N / 16;
     const uint32_t bx = (g.nrb + 3) / 4;
-    // A chunk's rows and a row block's tiles are addressed in 32 bits.
-    if ((uint64_t)g.x_stride * 64 * 2 >= (1ull << 32) || (uint64_t)g.kt * S * 4096 >= (1ull << 32))
-        return K3X_ERR_INVALID_EXTENT;
+    if (!dense_rows_addressable(g.x_stride, g.kt * S * 4096ull))
+        return launch_dense_passes<S, OUT, SPLIT>(ctx, g, N, stream);
     if (g.tokens <= 32)
         hipLaunchKernelGGL((dense_rows_kernel<S, 2, OUT, SPLIT>), dim3(bx), dim3(512), 0, stream,
                            g);
