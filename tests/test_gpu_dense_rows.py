@@ -1,6 +1,6 @@
 """The dense projections at the edges of the rows kernel's token tiles
 (pipeline.hip, dense_rows_kernel), and on either side of the GEMV's and the
-wide GEMM's ranges.
+wide GEMM's ranges (the wide GEMM's split kernels among them).
 
 * The layer's shared expert against float64, element-wise: the projections'
   fp32 sums within 2^-16 sum |w x| (at most 2304 terms of 2^-24, several times
@@ -46,7 +46,7 @@ def bits(t):
 
 
 @pytest.mark.parametrize("H,S", [(640, 384), (2304, 128)], ids=["few_tiles", "more_tiles_than_waves"])
-@pytest.mark.parametrize("T", [5, 16, 17, 32, 33, 64, 65, 127, 128])
+@pytest.mark.parametrize("T", [5, 16, 17, 32, 33, 64, 65, 127, 128, 193, 255, 256])
 @pytest.mark.parametrize("split_in", [False, True], ids=["bf16", "split_input"])
 def test_shared_expert_rows(hip, H, S, T, split_in):
     k3x, ctx = hip
@@ -87,11 +87,19 @@ def test_shared_expert_rows(hip, H, S, T, split_in):
     bank.close()
 
 
-@pytest.mark.parametrize("T", [17, 32, 33, 64, 65, 100])
-def test_official_rows_match_gemv(hip, T):
+# Shapes (H, L, I, Is, E, K): the second one's projections take the wide GEMM
+# from 256 tokens, and its experts the wide GEMM's split class kernels from 448
+# (at 460: chunks of 128 rows and last ones of 65 to 128).
+ROWS, WIDE = (1024, 2304, 128, 384, 8, 2), (1024, 512, 512, 512, 16, 8)
+
+
+@pytest.mark.parametrize("shape,T", [(ROWS, T) for T in (17, 32, 33, 64, 65, 100, 129, 200, 255)] +
+                         [(WIDE, T) for T in (17, 255, 256, 300, 460)],
+                         ids=lambda v: None if isinstance(v, int) else "rows" if v is ROWS else "wide")
+def test_official_rows_match_gemv(hip, shape, T):
     k3x, ctx = hip
-    H, L, I, Is, E, K = 1024, 2304, 128, 384, 8, 2
-    say(f"official rows T={T}")
+    H, L, I, Is, E, K = shape
+    say(f"official rows {shape} T={T}")
     bank = k3x.Bank(ctx, k3x.LayerShape(L, I, E, 0))
     bank.fill_synthetic(3, 119, 123)
     off = k3x.Official(ctx, bank, H, Is)

@@ -3,9 +3,9 @@
 * Top-K ties go to the lower expert index (runtime/src/official_moe.cpp:226-232,
   runtime/src/routing_policy.cpp:83-87), on every device Top-K: the decode
   path's select kernel (up to 512 experts), the general path's threshold
-  Top-K for few tokens (257 to 512 and 513 to 1024 experts), its register
-  Top-K with 4, 8 and 16 keys per lane (up to 256, 512 and 1024 experts; more
-  than 256 tokens past 256 experts) and the LDS Top-K past 1024 experts.  Two kinds of tie: every score equal (zero
+  Top-K (257 to 512 experts up to 256 tokens, 513 to 1024 at any), its register
+  Top-K with 4 and 8 keys per lane (up to 256 experts; 257 to 512 past 256
+  tokens) and the LDS Top-K past 1024 experts.  Two kinds of tie: every score equal (zero
   input, equal bias: ids 0..K-1, weights routed_scale / K), and planted groups
   of duplicated router rows with equal bias, within one lane and across
   lanes, straddling the K boundary (the lower ids are selected, in order).

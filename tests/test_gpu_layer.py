@@ -423,8 +423,8 @@ def test_router_shapes(hip, oracle, T, H, E):
 
 
 # Few tokens on the general path: the register router (one, two and four
-# token rows; the loop kernel past 8192 hidden) and the register Top-K (8 and
-# 16 keys per lane; the LDS kernel past 1024 experts), all bit-exact.
+# token rows; the loop kernel past 8192 hidden) and the threshold Top-K (512 and
+# 1024 experts; the LDS kernel past 1024), all bit-exact.
 @pytest.mark.parametrize("T,H,E", [(1, 1152, 1000), (2, 7168, 600), (3, 8192, 300),
                                    (4, 7168, 1030), (2, 8320, 700)],
                          ids=["t1", "t2", "t3", "t4_e1030", "t2_h8320"])
@@ -748,10 +748,9 @@ def test_c4_verification_window(hip, oracle, parity_report):
 
 
 # Verification windows between the decode path and the wide GEMM (4 < T <=
-# 64): the routed experts run on the decode gate/up and down kernels with a
-# slot's rows staged through LDS four at a time.  Cases: few rows per expert
-# (T=9); Zipf-skewed slots of many rows, most not a multiple of four (T=40);
-# I=3072, whose down projection holds 24 code tiles (T=64, 16 experts).
+# 64), on the streaming GEMM.  Cases: few rows per expert (T=9); Zipf-skewed
+# slots of many rows, most not a multiple of four (T=40); I=3072 (T=64, 16
+# experts).  Few pairs: tests/test_gpu_few_pairs.py.
 WINDOWS = {
     "t9": dict(tokens=9, hidden=1024, inter=512, experts=64, top_k=8, shared_inter=256),
     "t40_skew": dict(tokens=40, hidden=2048, inter=1024, experts=32, top_k=4, shared_inter=0,

@@ -78,9 +78,10 @@ def build(k3x_amd, ctx, oracle, shape, seed):
     return w, experts, bank, off
 
 
-# (H, L, I, Is, E): the second shape puts routed_down and the shared FFN on
-# the wide grouped GEMM from 128 tokens; the third has no shared FFN.
-# The fourth has enough experts for the 16-keys-per-lane Top-K, and for the
+# (H, L, I, Is, E): the second shape's projections run on the rows kernel from 17
+# tokens (the wide GEMM's ranges: tests/test_gpu_dense_rows.py and
+# tests/test_gpu_wide.py); the third has no shared FFN.
+# The fourth has enough experts for the 1024-expert threshold Top-K, and for the
 # few-token path (T <= 4: route, latent projection and shared FFN in two
 # launches); the fifth is that path without a shared FFN.  Few rows run the
 # projections as split-K GEMVs, 300 rows the router on the matrix cores.

@@ -5,8 +5,8 @@ Routes are given (k3x_hip_moe_forward_routed) so that each expert gets a
 chosen number of rows: around one row tile of 16, the 32, 48 and 64 rows of
 a chunk, and past it; K extents of one to a few tiles (not multiples of the
 ring), output row blocks that do not fill a workgroup, one slot a token and
-two, both record layouts (small routes and row chunks), and split input and
-activation rows.
+two, both record layouts (a slot an expert up to four tokens, row chunks beyond),
+experts of more rows than a pass, and split input and activation rows.
 
 Bounds, element-wise: a projection's fp32 sum is within 2^-16 sum |w x| of
 the float64 one (5 K tiles at most: 640 terms of 2^-24 each, doubled); the
@@ -54,7 +54,14 @@ CASES = {
     "chunks_split_both": (384, 640, EDGE, 1, True, True),
     "chunks_split_in": (384, 640, EDGE, 1, True, False),
     "one_chunked_expert": (512, 256, [0, 300, 0], 1, False, False),
-    "small_long": (256, 512, [1, 2, 100, 130], 1, False, False),  # 233 pairs: slot records
+    # T <= 4: the small-route grouping's slot records.
+    "slots_t4": (640, 384, [4, 3, 1], 2, False, False),
+    "slots_t3_split_act": (640, 384, [3, 2, 1], 2, False, True),
+    "slots_t4_split_both": (640, 384, [4, 0, 3, 1], 2, True, True),
+    # 65 to 96 tokens: two row tiles, busier experts in several passes.
+    "passes_t70": (640, 384, [33, 48, 64, 65], 3, False, False),
+    "passes_t70_split_act": (640, 384, [33, 48, 64, 65], 3, False, True),
+    "small_long": (256, 512, [1, 2, 100, 130], 1, False, False),
     "small_long_split": (256, 512, [1, 2, 100, 130], 1, True, True),
     "t16": (896, 128, [3, 4, 0, 9], 1, False, False),
     "t16_split": (896, 128, [3, 4, 0, 9], 1, True, True),
