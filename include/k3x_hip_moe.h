@@ -130,15 +130,15 @@ enum k3x_flags {
      * as bf16 hi + lo halves, [T][2 H] (hi = bf16(v), lo = bf16(v - hi)),
      * and the gate/up projections run over both halves; the latent layer's
      * fp32 experts (runtime/src/backend_cpu.cpp:317-318).  Runs the
-     * general path's narrow GEMMs. */
+     * general path's streaming GEMM. */
     K3X_FLAG_SPLIT_INPUT = 8u,
     /* Multiply the routed experts of the wide GEMM (prefill chunks, many
      * rows per expert) on the scaled FP4 MFMA: the bf16 activation rows are
      * re-encoded as two FP8 E4M3 terms with one power-of-two scale per 32
      * values each (exact for bf16 values down to 2^-13 of their block's
      * largest, within 2^-21 of it below), the MXFP4 weights go in as they
-     * are stored.  Ignored with K3X_FLAG_SPLIT_ACT and on the decode and
-     * narrow paths. */
+     * are stored.  Ignored with K3X_FLAG_SPLIT_ACT and below 128 tokens
+     * (the decode kernels and the streaming GEMM). */
     K3X_FLAG_SCALED_FP4 = 16u,
 };
 

@@ -68,9 +68,8 @@ constexpr int scale_step() {
 }
 
 // Vector-memory requests one wave issues at pipeline step k (AL of the
-// activation tile,
-// q8 scale dwords, weight tile; the MXFP4 scale dwords cover four K tiles and
-// are requested at steps with k % 4 == scale_step).
+// activation tile, q8 scale dwords, weight tile; the MXFP4 scale dwords cover
+// four K tiles and are requested at steps with k % 4 == scale_step).
 template <bool FP4, int NT, int S, int U, bool Q, int AL>
 constexpr int step_loads(int d) {
     return AL + (Q ? 1 : 0) + NT * S * U + ((FP4 && d == scale_step<Q>()) ? NT * S : 0);
@@ -279,10 +278,11 @@ __global__ __launch_bounds__(kThreads, 1) void wide_gemm(WideGemmArgs a) {
             (k) * 8, 0, 0);
 #define WIDE_ORDER() asm volatile("" ::: "memory")
 
-    // MT = row tiles multiplied: the chunk's rows rounded up to 32, 64, 96
-    // or 128 rows, see the dispatch at the end (a workgroup-uniform choice
-    // made once, so the step loop has no branches; tiles past the chunk's
-    // rows hold copies of its last row and are not stored).
+    // MT = row tiles multiplied: the launch's class, one fewer where a chunk
+    // of at most 64 rows allows it, or the shared kinds' four, six or eight; see
+    // the dispatch at the end (a workgroup-uniform choice made once, so the
+    // step loop has no branches; rows past the chunk's are copies of its last
+    // row and are not stored).
     auto run = [&](auto mt_count) {
         constexpr int MT = decltype(mt_count)::value;
         f32x4 acc[MT][NT][S];

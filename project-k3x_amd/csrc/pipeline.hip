@@ -1624,8 +1624,8 @@ template <int S, int MT, int OUT, bool SPLIT>
 __global__ __launch_bounds__(512, 1) void dense_rows_kernel(GemvArgs a) {
     constexpr uint32_t kStage = MT * 256;  // 16-byte words per ring stage
     constexpr uint32_t kRing = kRowsStages * kStage;
-    static_assert(8 * MT * S * 64 <= 2 * kRing || MT == 1, "the partial sums fit the rings");
-    __shared__ u32x4 s_a4[2 * kRing > 8 * MT * S * 64 ? 2 * kRing : 8 * MT * S * 64];
+    static_assert(8 * MT * S * 64 <= 2 * kRing, "the partial sums fit the rings");
+    __shared__ u32x4 s_a4[2 * kRing];
     if (*(volatile const uint32_t*)a.status) return;
     const uint32_t lane = threadIdx.x & 63;
     const uint32_t wv = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -2954,9 +2954,9 @@ int launch_topk(k3x_hip_ctx* ctx, const float* logits, const float* bias, uint32
     return launch_topk_any(ctx, logits, bias, E, K, T, routed_scale, renorm, ids, weights);
 }
 
-// Dense bf16 projections in the bank's tile layout: the wide grouped GEMM
-// (one item per 128-row chunk of the T rows) from kWideMinTokens rows when
-// the shapes fit it, else expert_gemm over the T rows as one block.
+// Dense bf16 projections in the bank's tile layout: the GEMV up to 16 rows,
+// the rows kernel above, and from kDenseWideTokens rows the wide grouped GEMM
+// (one item per 128-row chunk of the T rows) where the shapes fit it.
 // The wide GEMM's dense kinds: shapes, and the tokens from which they beat
 // the rows kernel.
 bool dense_wide_ok(WideKind kind, uint32_t N, uint32_t K, uint32_t T) {

@@ -1,6 +1,6 @@
 // stream_gemm.hip -- the streaming expert GEMM: experts with few rows (1 to
 // 64 a record), where the MXFP4 weights' stream from HBM bounds the launch
-// and the rows only ride along.
+// and the rows only ride along (which calls take it: k3x_select.hpp).
 //
 // Workgroup = 4 waves, one record (expert, up to kStreamRows rows; a record
 // with more is walked in chunks) x kRb 16-row output blocks, each wave its
@@ -24,7 +24,9 @@
 //   T=64 (24 at most)        gate/up 4.1 -> 6.5, down 4.8 -> 5.9
 //   T=127 (44 at most)       gate/up 3.9 -> 6.3, down 3.6 -> 5.8
 //   T=331 (97 at most)       gate/up 3.9 -> 5.3, down 3.8 -> 4.6
-// and with split down rows (3584 x 3072 experts) at T=97 2.6 -> 6.1.
+// and with split down rows (3584 x 3072 experts) at T=97 2.6 -> 6.1.  (Down at
+// one row tile is the one that lost; the gate/up of the same calls and their
+// shorter grouping gain several times that.)
 // Uniform 16, 32 and 64 rows an expert: 6.3, 5.5 and 4.1 TB/s gate/up.
 #include <hip/hip_runtime.h>
 
@@ -332,10 +334,13 @@ void launch(const StreamGemmArgs& a, uint32_t max_recs, hipStream_t stream) {
 }
 
 // MAXT by the most rows an expert can have, at most TMAX (records with more
-// rows are walked in chunks).  Two row tiles up to 96 tokens: few experts have
-// more than 32 rows there, and the others gain from three workgroups a CU
-// instead of two (T=64, two / four row tiles: gate/up 6.7 / 6.4 TB/s, down 6.2
-// / 5.8; T=97 6.5 / 6.2 and 6.0 / 5.8; T=127 6.0 / 6.35 and 5.7 / 5.8).
+// rows are walked in chunks).  Two row tiles up to 96 tokens: few of many experts
+// have more than 32 rows there, and the others gain from three workgroups a CU
+// instead of two.  384 experts, Top-16, layer us with two / four row tiles: T=64
+// 687 / 693, 80 738 / 742, 96 754 / 766; level from there (97 730 / 733, 104 778
+// / 771, 112 786 / 800), then four (120 812 / 784, 127 884 / 835).  Few busy
+// experts would want four earlier (16 experts Top-8: T=48 119 / 118, 64 166 / 132,
+// 96 233 / 183).
 template <bool GATEUP, bool SPLITIN, bool SPLITOUT, int TMAX>
 void launch_tiles(const StreamGemmArgs& a, uint32_t max_recs, uint32_t max_rows,
                   hipStream_t stream) {
