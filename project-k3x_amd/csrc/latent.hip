@@ -43,7 +43,8 @@ __device__ inline float situ(float g, float u, float beta, int has_linear, float
 }
 
 // One output row per wave, T <= kMaxTokens tokens per pass (x rows
-// [T][x_stride]): shapes that the vector kernel below does not take.
+// [T][x_stride]): shapes that the vector kernel below does not take, and (VEC:
+// 16-byte loads, cols % 4 == 0, rows 16-byte aligned) columns too short for it.
 // OUT: 0 y = Wx; 1 y = Wx + add (fp32 add, as routed[row] += shared[row]);
 // 2 y = Wx and the split copy ys = [bf16 hi | bf16 lo] rows of 2 rows_total;
 // 3 y = situ(W x, W2 x) (the gate / up pair of an MLP).
@@ -63,7 +64,7 @@ struct GemvArgs {
     const uint32_t* status;
 };
 
-template <int OUT>
+template <int OUT, bool VEC>
 __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
     if (*(volatile const uint32_t*)a.status) return;
     const uint32_t lane = threadIdx.x & 63;
@@ -80,16 +81,50 @@ __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
         for (int m = 0; m < M; ++m)
 #pragma unroll
             for (uint32_t t = 0; t < kMaxTokens; ++t) acc[m][t] = 0.0;
-        for (uint32_t c = lane; c < a.cols; c += 64) {
-            float w[M];
+        if constexpr (VEC) {
+            // Four 16-byte loads per lane in flight (4 KiB per wave).
+            constexpr uint32_t kStep = 64 * 4 * 4;
+            for (uint32_t c0 = 0; c0 < a.cols; c0 += kStep) {
+                f32x4 w[M][4];
 #pragma unroll
-            for (int m = 0; m < M; ++m) w[m] = wr[m][c];
+                for (int m = 0; m < M; ++m)
 #pragma unroll
-            for (uint32_t t = 0; t < kMaxTokens; ++t) {
-                if (t >= nt) break;
-                const double xv = (double)a.x[(size_t)(t0 + t) * a.x_stride + c];
+                    for (int q = 0; q < 4; ++q) {
+                        const uint32_t c = c0 + (q * 64 + lane) * 4;
+                        w[m][q] = c < a.cols ? *reinterpret_cast<const f32x4*>(wr[m] + c)
+                                             : f32x4{0.f, 0.f, 0.f, 0.f};
+                    }
 #pragma unroll
-                for (int m = 0; m < M; ++m) acc[m][t] = __builtin_fma((double)w[m], xv, acc[m][t]);
+                for (uint32_t t = 0; t < kMaxTokens; ++t) {
+                    if (t >= nt) break;
+                    const float* xr = a.x + (size_t)(t0 + t) * a.x_stride;
+#pragma unroll
+                    for (int q = 0; q < 4; ++q) {
+                        const uint32_t c = c0 + (q * 64 + lane) * 4;
+                        if (c >= a.cols) continue;
+                        const f32x4 xv = *reinterpret_cast<const f32x4*>(xr + c);
+#pragma unroll
+                        for (int i = 0; i < 4; ++i)
+#pragma unroll
+                            for (int m = 0; m < M; ++m)
+                                acc[m][t] =
+                                    __builtin_fma((double)w[m][q][i], (double)xv[i], acc[m][t]);
+                    }
+                }
+            }
+        } else {
+            for (uint32_t c = lane; c < a.cols; c += 64) {
+                float w[M];
+#pragma unroll
+                for (int m = 0; m < M; ++m) w[m] = wr[m][c];
+#pragma unroll
+                for (uint32_t t = 0; t < kMaxTokens; ++t) {
+                    if (t >= nt) break;
+                    const double xv = (double)a.x[(size_t)(t0 + t) * a.x_stride + c];
+#pragma unroll
+                    for (int m = 0; m < M; ++m)
+                        acc[m][t] = __builtin_fma((double)w[m], xv, acc[m][t]);
+                }
             }
         }
 #pragma unroll
@@ -123,6 +158,9 @@ __global__ __launch_bounds__(kThreads) void f32_gemv_kernel(GemvArgs a) {
 // by the workgroup, are read and converted to double once for both; the
 // weights are non-temporal (read once a call) and eight 16-byte loads a lane
 // are in flight.  Lane l sums columns 4 (64 i + l) .. + 3, i ascending.
+// The tail of a row has a body of its own, so that the full steps carry no bounds
+// (384 x 7168, one token 10.9 -> 9.5 us, 36 x 7168 10.6 -> 9.4; the latent layer at 8
+// tokens 254 -> 246).
 // Bound: HBM.  Measured (7168 columns, one token) against a row a wave with x
 // read from the cache beside every weight: the gate/up of 6144 rows and a
 // 3584-row matrix 3.5 and 3.2 TB/s in two launches, 6.6 in one; two down
@@ -160,55 +198,62 @@ struct VecArgs {
 
 constexpr uint32_t kCols = 1024;
 
-// acc[r][t] += w[r] . x[t] over cols columns, by the whole workgroup.
+// acc[r][t] += w[r] . x[t] over the columns from c0, by the whole workgroup: kCols
+// of them (FULL) or the cols - c0 that are left, whose absent quarters of 256
+// are neither loaded nor multiplied.
+template <int NT, bool FULL>
+__device__ __forceinline__ void dot_block(const float* const (&w)[2], uint32_t c0, uint32_t cols,
+                                          const float* x, uint32_t x_stride, uint32_t nt,
+                                          f32x4 (&s_x)[NT][kCols / 4], double (&acc)[2][NT]) {
+    const uint32_t lane = threadIdx.x & 63;
+    const uint32_t cx = c0 + threadIdx.x * 4;
+    const uint32_t quarters = FULL ? 4 : (cols - c0 + 255) / 256;  // workgroup-uniform
+    f32x4 xv[NT], wv[2][4];
+#pragma unroll
+    for (int t = 0; t < NT; ++t)
+        xv[t] = (FULL || cx < cols) && (uint32_t)t < nt
+                    ? *reinterpret_cast<const f32x4*>(x + (size_t)t * x_stride + cx)
+                    : f32x4{0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+    for (int r = 0; r < 2; ++r)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            const uint32_t c = c0 + (q * 64 + lane) * 4;
+            if constexpr (FULL)
+                wv[r][q] = __builtin_nontemporal_load(reinterpret_cast<const f32x4*>(w[r] + c));
+            else
+                wv[r][q] = c < cols ? *reinterpret_cast<const f32x4*>(w[r] + c)
+                                    : f32x4{0.f, 0.f, 0.f, 0.f};
+        }
+    // The barriers wait for LDS only: the weights stay in flight.
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < NT; ++t) s_x[t][threadIdx.x] = xv[t];
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+#pragma unroll
+    for (int t = 0; t < NT; ++t) {
+        if (!FULL && (uint32_t)t >= nt) break;
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (!FULL && (uint32_t)q >= quarters) break;
+            const f32x4 v = s_x[t][q * 64 + lane];
+#pragma unroll
+            for (int i = 0; i < 4; ++i)
+#pragma unroll
+                for (int r = 0; r < 2; ++r)
+                    acc[r][t] = __builtin_fma((double)wv[r][q][i], (double)v[i], acc[r][t]);
+        }
+    }
+}
+
 template <int NT>
 __device__ inline void dot_rows(const float* const (&w)[2], uint32_t cols, const float* x,
                                 uint32_t x_stride, uint32_t nt, f32x4 (&s_x)[NT][kCols / 4],
                                 double (&acc)[2][NT]) {
-    const uint32_t lane = threadIdx.x & 63;
-    for (uint32_t c0 = 0; c0 < cols; c0 += kCols) {
-        const uint32_t cx = c0 + threadIdx.x * 4;
-        f32x4 xv[NT], wv[2][4];
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-            xv[t] = cx < cols && (uint32_t)t < nt
-                        ? *reinterpret_cast<const f32x4*>(x + (size_t)t * x_stride + cx)
-                        : f32x4{0.f, 0.f, 0.f, 0.f};
-        if (c0 + kCols <= cols) {
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int q = 0; q < 4; ++q)
-                    wv[r][q] = __builtin_nontemporal_load(
-                        reinterpret_cast<const f32x4*>(w[r] + c0 + (q * 64 + lane) * 4));
-        } else {
-#pragma unroll
-            for (int r = 0; r < 2; ++r)
-#pragma unroll
-                for (int q = 0; q < 4; ++q) {
-                    const uint32_t c = c0 + (q * 64 + lane) * 4;
-                    wv[r][q] = c < cols ? *reinterpret_cast<const f32x4*>(w[r] + c)
-                                        : f32x4{0.f, 0.f, 0.f, 0.f};
-                }
-        }
-        // The barriers wait for LDS only: the weights stay in flight.
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-        for (int t = 0; t < NT; ++t) s_x[t][threadIdx.x] = xv[t];
-        asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
-#pragma unroll
-        for (int t = 0; t < NT; ++t)
-#pragma unroll
-            for (int q = 0; q < 4; ++q) {
-                const f32x4 v = s_x[t][q * 64 + lane];
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int r = 0; r < 2; ++r)
-                        acc[r][t] =
-                            __builtin_fma((double)wv[r][q][i], (double)v[i], acc[r][t]);
-            }
-    }
+    uint32_t c0 = 0;
+    for (; c0 + kCols <= cols; c0 += kCols)
+        dot_block<NT, true>(w, c0, cols, x, x_stride, nt, s_x, acc);
+    if (c0 < cols) dot_block<NT, false>(w, c0, cols, x, x_stride, nt, s_x, acc);
 }
 
 template <int NT>
@@ -405,12 +450,26 @@ int launch_vec(k3x_hip_ctx* ctx, const VecJob& a, const VecJob* b, uint32_t T) {
     return launched(ctx, 1);
 }
 
-template <int OUT>
+template <int OUT, bool VEC = false>
 int launch_gemv(k3x_hip_ctx* ctx, GemvArgs a, hipStream_t stream) {
     a.status = ctx->status;
-    hipLaunchKernelGGL(f32_gemv_kernel<OUT>, dim3((a.rows + kWaves - 1) / kWaves), dim3(kThreads),
-                       0, stream, a);
+    hipLaunchKernelGGL((f32_gemv_kernel<OUT, VEC>), dim3((a.rows + kWaves - 1) / kWaves),
+                       dim3(kThreads), 0, stream, a);
     return launched(ctx, 1);
+}
+
+// Whether a product alone runs a row a wave instead of the vector kernel's two,
+// whose staging of 1024 columns and sums over a pass of eight tokens outweigh
+// short rows' loads: up to 768 columns, but only to 512 where the passes are full and x
+// is another kernel's output of this call (x_new), which every wave would fetch for
+// itself from beyond its L2.  us, row a wave / vector: 7168 rows of 64 columns, 1 token
+// 4.4 / 4.4, 5 8.0 / 14.9, 9 12.2 / 26.9; 4096 x 512, 5 tokens 7.7 / 9.6, 8 9.3 / 10.1;
+// 4096 x 768, 9 tokens 12.1 / 15.8; 512 x 768, 8 tokens 7.4 / 8.3, 16 12.8 / 14.3, and
+// as the down product of an MLP of 1024 columns, with its gate / up, 22.1 / 19.7 and
+// 38.2 / 33.6; 4096 x 1024, 5 tokens 11.8 / 9.9.  (The latent layer's paired products
+// keep the vector kernel: a launch less is worth more there.)
+bool short_cols(uint32_t cols, uint32_t T, bool x_new) {
+    return cols <= (T % 8 == 0 && x_new ? 512u : 768u);
 }
 
 VecJob plain_job(const float* W, uint32_t rows, uint32_t cols, const float* x, float* y) {
@@ -440,12 +499,14 @@ GemvArgs plain_args(const float* W, uint32_t rows, uint32_t cols, const float* x
     return a;
 }
 
-// y = W x.
+// y = W x; x_new: x is written by a kernel of the same call.
 int matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, uint32_t cols, const float* x,
-           uint32_t T, float* y) {
-    if (vec_ok(W, x, cols, cols))
-        return launch_vec(ctx, plain_job(W, rows, cols, x, y), nullptr, T);
-    return launch_gemv<0>(ctx, plain_args(W, rows, cols, x, T, y), ctx->stream);
+           uint32_t T, float* y, bool x_new) {
+    if (!vec_ok(W, x, cols, cols))
+        return launch_gemv<0>(ctx, plain_args(W, rows, cols, x, T, y), ctx->stream);
+    if (short_cols(cols, T, x_new))
+        return launch_gemv<0, true>(ctx, plain_args(W, rows, cols, x, T, y), ctx->stream);
+    return launch_vec(ctx, plain_job(W, rows, cols, x, y), nullptr, T);
 }
 
 // act = situ(gate x, up x) as a vector job.
@@ -468,7 +529,8 @@ bool situ_vec_ok(const float* gate, const float* up, const float* x, uint32_t co
 int situ_product(k3x_hip_ctx* ctx, const float* gate, const float* up, uint32_t rows,
                  uint32_t cols, const float* x, uint32_t T, float* act, float beta, bool has_linear,
                  float linear) {
-    if (situ_vec_ok(gate, up, x, cols))
+    const bool vec = situ_vec_ok(gate, up, x, cols);
+    if (vec && !short_cols(cols, T, false))
         return launch_vec(ctx, situ_job(gate, up, rows, cols, x, act, beta, has_linear, linear),
                           nullptr, T);
     GemvArgs g = plain_args(gate, rows, cols, x, T, act);
@@ -476,7 +538,7 @@ int situ_product(k3x_hip_ctx* ctx, const float* gate, const float* up, uint32_t 
     g.beta = beta;
     g.has_linear = has_linear;
     g.linear = linear;
-    return launch_gemv<3>(ctx, g, ctx->stream);
+    return vec ? launch_gemv<3, true>(ctx, g, ctx->stream) : launch_gemv<3>(ctx, g, ctx->stream);
 }
 
 bool dims_ok(uint32_t rows, uint32_t cols, uint32_t T) {
@@ -508,7 +570,7 @@ int k3x_hip_dense_f32_matvec(k3x_hip_ctx* ctx, const float* W, uint32_t rows, ui
                              const float* x, uint32_t tokens, float* y) {
     if (!ctx || !W || !x || !y || !dims_ok(rows, cols, tokens)) return K3X_ERR_INVALID_EXTENT;
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
-    return matvec(ctx, W, rows, cols, x, tokens, y);
+    return matvec(ctx, W, rows, cols, x, tokens, y, false);
 }
 
 int k3x_hip_mxfp4_matvec(k3x_hip_ctx* ctx, const uint8_t* packed, const uint8_t* scales,
@@ -533,7 +595,7 @@ int k3x_hip_dense_situ_mlp(k3x_hip_ctx* ctx, const float* gate, const float* up,
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
     const int st = situ_product(ctx, gate, up, inter, hidden, x, tokens, act, situ_beta,
                                 has_situ_linear != 0, situ_linear_beta);
-    return st ? st : matvec(ctx, down, out_rows, inter, act, tokens, y);
+    return st ? st : matvec(ctx, down, out_rows, inter, act, tokens, y, true);
 }
 
 int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
@@ -626,7 +688,7 @@ int k3x_hip_resident_moe_layer(k3x_hip_ctx* ctx, k3x_hip_bank* bank,
         o.x2_stride = S;
         return launch_vec(ctx, o, nullptr, T);
     }
-    if ((st = matvec(ctx, w->routed_up, H, L, normed, T, routed))) return st;
+    if ((st = matvec(ctx, w->routed_up, H, L, normed, T, routed, true))) return st;
     if (down_vec) {
         VecJob o = plain_job(w->shared_down, H, S, sact, out);
         o.out = kOutAdd;

@@ -1,6 +1,6 @@
-"""The vector form of the fp32 products (latent.hip) at its edges: odd row
-counts, columns short of, at and past the staged 1024, one token to more than
-a pass of eight; against float64 rounded once.  Sums are formed in double, so
+"""The fp32 products (latent.hip) at their edges: odd row counts, columns short of,
+at and past the staged 1024 and the quarters of its tail, on either side of the
+short rows' own kernel (512, 768 columns), one token to more than a pass of eight; against float64 rounded once.  Sums are formed in double, so
 every output is within one fp32 ulp (2^-23 of its value at most, plus 2^-40 of
 sum |w x| where the terms cancel)."""
 from __future__ import annotations
@@ -27,7 +27,8 @@ def rand(g, *shape):
     return torch.randn(shape, device="cuda:0", generator=g)
 
 
-@pytest.mark.parametrize("rows,cols", [(1, 4), (2, 1020), (37, 1024), (129, 1028), (8, 3072)])
+@pytest.mark.parametrize("rows,cols", [(1, 4), (2, 1020), (37, 1024), (129, 1028), (8, 3072), (5, 512), (7, 516),
+                                       (9, 768), (6, 772), (3, 1280), (11, 1796)])
 @pytest.mark.parametrize("T", [1, 2, 3, 4, 5, 8, 9, 17])
 def test_matvec_edges(hip, rows, cols, T):
     k3x, ctx = hip
@@ -50,6 +51,8 @@ def test_situ_mlp_odd_rows(hip, T):
     are about an ulp off each: 2^-20 of the activation covers them."""
     k3x, ctx = hip
     H, I, O = 1028, 36, 35
+    if T == 4:
+        H, I = 260, 772  # gate and up a row a wave, down in the vector form
     g = torch.Generator(device="cuda:0")
     g.manual_seed(T)
     gate, up, down = rand(g, I, H) * 0.05, rand(g, I, H) * 0.05, rand(g, O, I) * 0.2
