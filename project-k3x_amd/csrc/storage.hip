@@ -45,6 +45,7 @@ constexpr int kTables = 3 + kLevels;     // LDS: slicing, the tree levels, advan
 constexpr int kSub = 4, kBigSub = 16;    // 4 KiB sub-chunks of a wave's chunk, and of a big
                                          // buffer's
 constexpr size_t kBigBytes = 32u << 20;
+constexpr size_t kHostBytes = 1024;      // k3x_hip_crc32c: below, the host folds the bytes
 constexpr int kAdvLevels = 40;           // advance tables: 64 * 2^k bytes
 constexpr int kCrcThreads = 256;
 
@@ -316,9 +317,13 @@ int crc32c_device(k3x_hip_ctx* ctx, const void* data, size_t bytes, uint32_t* cr
     if (!ctx || (!data && bytes) || !crc) return K3X_ERR_INVALID_EXTENT;
     if (reinterpret_cast<uintptr_t>(data) % 16) return K3X_ERR_INVALID_EXTENT;
     if (hipSetDevice(ctx->device) != hipSuccess) return K3X_ERR_BACKEND_UNAVAILABLE;
-    // Whole 16-byte words on the device, the tail on the host.
-    const size_t body = bytes & ~(size_t)15, tail = bytes % 16;
-    uint8_t tail_bytes[16];
+    // Whole 16-byte words on the device, the tail on the host; a few bytes, or a
+    // tail beside a few more, wholly there: one small copy, no launch (us, host /
+    // device: 100 bytes 21.6 / 32.8, 512 22.4 / 23.6, 4095 28.2 / 33.1; 2048
+    // 25.0 / 23.6).
+    const bool host = bytes < kHostBytes || (bytes < kChunk && bytes % 16);
+    const size_t body = host ? 0 : bytes & ~(size_t)15, tail = bytes - body;
+    uint8_t tail_bytes[kChunk];
     if (body) {
         const Extent e{data, body, 0, false};
         if (int st = launch_extent_check(ctx, &e, 1)) return st;

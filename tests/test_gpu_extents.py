@@ -1,7 +1,7 @@
 """The one-launch extent check (storage.hip) at the edges of its chunks, and
 the device admission that rests on it (k3x_hip_bank_upload_expert_device).
 
-CRCs over sizes around a lane's words, a wave's 16 KiB, a workgroup's 64 KiB
+CRCs over sizes around what the host folds itself, a lane's words, a wave's 16 KiB, a workgroup's 64 KiB
 and the step to 64 KiB chunks at 32 MiB, against the oracle's CRC32C.  An
 admission with one extent corrupted, or a 0xFF byte in one array of scales,
 is refused with that extent's code before the slot is touched, in the order
@@ -28,7 +28,7 @@ def hip():
     ctx.close()
 
 
-@pytest.mark.parametrize("n", [32, 4080, 16384 - 16, 16384, 16384 + 16, 65536 - 16, 65536,
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 32, 1008, 1023, 1024, 1025, 4079, 4080, 4095, 4096, 4097, 16384 - 16, 16384, 16384 + 16, 65536 - 16, 65536,
                                65536 + 31, 64 * 16384, 65 * 16384 + 16, (1 << 20) + 7,
                                (32 << 20) - 16, 32 << 20, (32 << 20) + 65536 + 5])
 def test_crc_chunk_edges(hip, oracle, n):
@@ -38,6 +38,19 @@ def test_crc_chunk_edges(hip, oracle, n):
     dev = torch.from_numpy(host).to("cuda:0")
     st, crc = ctx.crc32c(dev, n)
     assert st == 0 and crc == oracle.crc32c(host.tobytes())
+
+
+def test_crc_of_few_bytes_takes_no_launch(hip, oracle):
+    """Below 1 KiB, and below 4 KiB with a tail, the bytes are copied and folded on
+    the host: a launch and a second copy would take half as long again."""
+    _, ctx = hip
+    host = np.random.default_rng(4).integers(0, 256, 4096, dtype=np.uint8)
+    dev = torch.from_numpy(host).to("cuda:0")
+    for n, launches in ((100, 0), (512, 0), (1023, 0), (1024, 1), (1030, 0), (4095, 0), (4096, 1)):
+        before = ctx.stats().kernel_launches
+        st, crc = ctx.crc32c(dev, n)
+        assert st == 0 and crc == oracle.crc32c(host[:n].tobytes()), n
+        assert ctx.stats().kernel_launches - before == launches, n
 
 
 def test_admission_refusals(hip, oracle):
