@@ -2,7 +2,7 @@
 """Writes the golden vectors under tests/golden/ from the reference's own CPU
 functions (oracle/_ref/libk3x_ref.so, compiled in place from the reference
 sources by `make -C oracle ref`).  Run in the container that holds the
-reference tree; the GPU box only reads the .npz files.
+reference tree; tests read the .npz files only.
 
 Inputs come from the build's seeded generator (tests/synth.py), so every
 fixture is regenerated bit-identically from its seed.

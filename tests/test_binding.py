@@ -6,7 +6,7 @@ an abstract or mismatched one fails to build).  Linked with the reference's
 CPU backend sources, it keeps the reference's error contract: only a shape
 the library declines before any device work runs on make_cpu_backend() (and
 is counted); a device failure is returned as a failure.  CPU only; skipped
-where the reference tree is absent (the GPU box)."""
+where the reference tree is absent."""
 from __future__ import annotations
 
 import os
